@@ -16,8 +16,28 @@
 // moves on to the next.  Device-scope atomics on one address serialise, so
 // spreading them over eight counters and claiming kClaim rays (2 per lane)
 // at a time keeps the counters off the critical path (the path tracer's
-// launches hold up to 5 rays per path, most of them short).  Two ray
-// sources:
+// launches hold up to 5 rays per path, most of them short).
+//
+// A launch of at most kSpreadRays rays per wave takes no claims: every wave
+// has one fixed window.  What bounds it is not throughput but the round
+// trips of its longest rays (p99.9 is 73 steps on the 1.3M-triangle mesh
+// where the mean is 10, about 1 us each) and, with claims, the counters:
+// every wave ends by finding all eight used up, 8 x 8,192 atomics of about
+// 12 ns per address.  The windows are as narrow as kSpreadWaves waves allow
+// (8 per CU, two per SIMD: 1,000 rays are traced one to a wave, where no
+// lane waits for another's branches), then kSpreadWindow rays wide (a lane
+// takes two, so refills keep the lanes busy), then as wide as the grid
+// makes them.  On the 100k-triangle sphere (claims of 128 before -> now):
+// 1,000 rays over 5k triangles 70 -> 38 us, 131k rays 165 -> 137, 400k
+// 262 -> 171, 1M 341 -> 237, 2M 400 -> 321; 500k any-hit rays 299 -> 200;
+// the 97x61 one-sample frame 1,087 -> 634 us.  At 4M rays (more than
+// kSpreadRays per wave) the two measured alike, and at 16M fixed windows
+// lose: waves that draw long rays end late.  kSpreadWaves 256 / 1,024 /
+// 4,096 / 8,192 instead of 2,048: 109 / 106 / 102 / 105 against 101 us at
+// 20k rays, the frame 720 / 659 / 615 / 610 against 635; windows of 64 or
+// 256 were 2-5% slower at 700k to 1M rays.
+//
+// Two ray sources:
 //   * SEG = false: rays[0, n) with n known to the host;
 //   * SEG = true : three segments whose sizes live in device memory (the
 //     path tracer's compacted continuation rays [0, cnt[0]), its next-event
@@ -33,6 +53,9 @@ namespace mcrt
 {
 constexpr int kWave = 64;
 constexpr uint32_t kClaim = 128;
+constexpr uint32_t kSpreadRays = 256;    // most rays per wave of a launch with fixed windows
+constexpr uint32_t kSpreadWaves = 2048;  // waves a small launch is spread over
+constexpr uint32_t kSpreadWindow = 128;  // widest window while fewer waves than the grid's suffice
 // Word of a segment-mode count array holding the third segment's size (on
 // its own 128 B line: the path tracer takes it with its own atomic).
 constexpr int kSeg2Word = 32;
@@ -86,7 +109,6 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     TraceCount cnt;
     uint32_t nrays = 0;
     const uint32_t lane = threadIdx.x;
-    const uint64_t below = lane == 0 ? 0ull : (~0ull >> (64u - lane));  // lanes under this one
     Tracer<ANY, COUNT> tr;
     SceneRoot root;
     root.nodes = S.nodes;
@@ -109,7 +131,19 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     // claim bookkeeping stays in scalar registers instead of being shuffled
     // through the LDS crossbar into vector registers.
     uint32_t ahead = 0;  // lane 0: offset of the requested next window in slice sl
-    if (lane == 0) ahead = atomicAdd(wq + sl * kSliceStride, kClaim);
+    if (total <= gridDim.x * kSpreadRays)
+    {
+        // a fixed window; past its end the wave finds its slice, the last
+        // one left to try, used up
+        const uint32_t need = (total + gridDim.x - 1) / gridDim.x;  // the windows cover every ray
+        const uint32_t win = max(need, min((total + kSpreadWaves - 1) / kSpreadWaves, kSpreadWindow));
+        claim = min(blockIdx.x * win, total);
+        claim_end = min(claim + win, total);
+        ahead = ~0u;
+        tried = kSlices - 1;
+    }
+    else if (lane == 0)
+        ahead = atomicAdd(wq + sl * kSliceStride, kClaim);
     const uint32_t refill = (uint32_t)S.refill_lanes;  // 1..64
     for (;;)
     {
@@ -143,7 +177,9 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                 claim_end = len - c < kClaim ? lo + len : lo + c + kClaim;
             }
             const uint32_t avail = claim_end - claim;
-            const uint32_t rank = (uint32_t)__popcll(idle & below);
+            // idle lanes under this one
+            const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
             if (!live && rank < avail)
             {
                 const uint32_t k = claim + rank;
@@ -184,12 +220,14 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     }
 }
 
-// Workgroups a trace launch uses: enough to cover n rays, at most the
-// number of lanes the spill buffer covers.
+// Workgroups a trace launch uses: enough to cover n rays and to spread few
+// of them over kSpreadWaves waves, at most the number of lanes the spill
+// buffer covers.
 inline int64_t trace_blocks(const DevScene& s, int64_t n)
 {
     int64_t max_blocks = s.spill_lanes / kWave;
     int64_t blocks = (n + kWave - 1) / kWave;
+    if (blocks < kSpreadWaves) blocks = n < kSpreadWaves ? n : kSpreadWaves;
     if (blocks > max_blocks) blocks = max_blocks;
     if (blocks < 1) blocks = 1;
     return blocks;

@@ -258,3 +258,24 @@ def test_ties_and_degenerate_triangles(ctx):
     tied = ((oprim >= 0) & (oprim < 50)) | ((oprim >= 100) & (oprim < 140)) | ((oprim >= 800) & (oprim < 890))
     assert tied.sum() > 500
     s.close()
+
+
+@pytest.mark.parametrize("n", [2, 63, 2047, 2049, 3000, 256 * 128 + 1, 256 * 256 - 1, 256 * 256, 256 * 256 + 1])
+def test_fixed_windows_and_claims_bit_exact(ctx, n):
+    """Launches with one fixed window per wave (at most 256 rays per wave of
+    the grid, here 256 waves) and with claimed windows, at the edges of the
+    window rule: every ray is traced once, closest and any hit."""
+    import mcrt_amd
+    print(f"[windows] n={n}", flush=True)
+    tris = _libs.debug_mesh()
+    s = mcrt_amd.Scene(ctx)
+    s.add(tris, s.add_material(mcrt_amd.DIFF, (0.5, 0.5, 0.5)))
+    s.set_tuning(trace_waves_per_cu=1)
+    s.finalize()
+    rays = _libs.random_rays(tris, n, seed=n)
+    want = _libs.OracleBVH(tris).intersect(rays)
+    for _ in range(2):
+        prim, tuv = mcrt_amd.split_hits(s.intersect(rays, np.full((n, 4), -7, np.int32)))
+        assert np.array_equal(prim, want[0])
+        assert np.array_equal(tuv.view(np.uint32), want[1].view(np.uint32))
+        assert np.array_equal(s.occluded(rays, np.full(n, 7, np.uint8)), (want[0] >= 0).astype(np.uint8))
