@@ -159,7 +159,7 @@ struct CacheHeader
     uint64_t tree_digest, payload_hash;
 };
 const char kCacheMagic[8] = {'M', 'C', 'R', 'T', 'B', 'V', 'H', '\0'};
-const uint32_t kCacheVersion = 2;  // 2: rank tables, single-reference children
+const uint32_t kCacheVersion = 3;  // 3: the nodes of optimize_wide
 
 // FNV-1a over 64-bit words (bytes beyond a multiple of 8 folded in last).
 uint64_t hash_bytes(const void* p, size_t n, uint64_t h = 0xcbf29ce484222325ull)
@@ -321,6 +321,7 @@ int finalize_scene(mcrt_scene* s, int threads, const char* cache)
         st.tree_digest = tree_digest(bt);
         collapse_wide(bt, s->tris, wb);
         { BTree().nodes.swap(bt.nodes); std::vector<SRef>().swap(bt.refs); }
+        optimize_wide(wb);
         std::vector<WNode>().swap(wb.nodes);
         if (cache)
         {

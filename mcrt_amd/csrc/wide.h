@@ -21,6 +21,13 @@ void collapse_wide(const BTree& bt, const std::vector<Tri>& tris, WideBVH& out);
 // Fills out.qnodes from out.nodes (collapse_wide calls it).
 void quantize_nodes(WideBVH& out);
 
+// Re-forms the nodes of a collapsed BVH (and orders its references to match)
+// for the fewest expected traversal steps.  The binary order that the rank
+// tables hold is kept down to single references, and every child box is the
+// union of its references' clipped boxes, so the tests that collapsing may
+// drop or add are the implied ones and results do not change.
+void optimize_wide(WideBVH& wb);
+
 // An upper bound, over every node and axis, of |origin| + 255 * scale (so
 // of the magnitude of every decoded plane and of 255 quantisation steps):
 // the scale of the rounding-error margin of the kernels' node tests

@@ -66,6 +66,21 @@ extern "C" void* emu_build(const float* v9, long long n, int threads)
     return e;
 }
 
+// The nodes re-formed as finalize does (optimize_wide); stats[5..7] follow.
+extern "C" void emu_optimize(void* h, long long* stats)
+{
+    Emu* e = (Emu*)h;
+    optimize_wide(e->wb);
+    if (!device_records(e->wb, e->recs)) return;
+    const size_t nq = e->recs.size();
+    e->recs.resize(nq + e->wb.refs.size());
+    if (!e->wb.refs.empty()) std::memcpy(&e->recs[nq], e->wb.refs.data(), e->wb.refs.size() * sizeof(WRef));
+    e->stats[5] = (long long)e->wb.nodes.size();
+    e->stats[6] = e->wb.stack_bound;
+    e->stats[7] = e->wb.depth;
+    for (int k = 0; k < 8; k++) stats[k] = e->stats[k];
+}
+
 extern "C" unsigned long long emu_digest(void* h, long long* stats)
 {
     Emu* e = (Emu*)h;

@@ -225,3 +225,47 @@ def test_node_margin_bounds_reference_planes(emu):
     assert 0.05 < worst.value < 0.75
     emu.emu_margin_check(400_000, 7, 0.125, out, ctypes.byref(worst))
     assert out[1] > 0
+
+
+@pytest.mark.parametrize("which", ["debug_mesh", "soup_slice", "cornell_displaced_f40", "coplanar", "line", "single"])
+def test_optimised_nodes_keep_every_hit(emu, which):
+    """The nodes that finalize traverses (optimize_wide): hits and t/u/v equal
+    the oracle's bit for bit with a shallow and a deep stack, any hit too,
+    the Moller-Trumbore tests are the reference's, no more references are
+    fetched than the collapse fetches, and every decoded plane contains its
+    child's box."""
+    rng = np.random.default_rng(5)
+    if which == "debug_mesh":
+        tris = _libs.debug_mesh()
+    elif which == "soup_slice":
+        tris = _libs.soup_slice()
+    elif which == "cornell_displaced_f40":
+        from mcrt_amd import scenes
+        tris = scenes.cornell_displaced(geodesic_freq=40).tris
+    elif which == "coplanar":  # flat boxes, repeated triangles
+        g = rng.uniform(0, 1, (300, 3, 3)).astype(np.float32)
+        g[..., 2] = 0.25
+        tris = np.concatenate([g, g[:40]]).reshape(-1, 9)
+    elif which == "line":      # every box area is 0
+        g = np.zeros((200, 3, 3), np.float32)
+        g[..., 0] = rng.uniform(0, 1, (200, 3))
+        tris = g.reshape(-1, 9)
+    else:
+        tris = rng.uniform(0, 1, (1, 9)).astype(np.float32)
+    rays = _libs.random_rays(tris, 1 << 12, seed=6)
+    e = Emu(tris)
+    _, before = e.trace(rays)
+    st = np.zeros(8, np.int64)
+    e.L.emu_optimize(e.h, ptr(st))
+    prim, tuv, oc = _libs.OracleBVH(tris).intersect(rays, counters=True)
+    for lds in (2, 16):
+        hits, cnt = e.trace(rays, lds=lds)
+        assert np.array_equal(hits[:, 0], prim)
+        assert np.array_equal(hits[:, 1:].view(np.uint32), tuv.view(np.uint32))
+    occ, _ = e.trace(rays, any_hit=True)
+    assert np.array_equal(occ, (prim >= 0).astype(np.uint8))
+    assert cnt[2] == oc[2]
+    assert cnt[1] <= before[1]
+    out = np.zeros(4, np.int64)
+    e.L.emu_check_qnodes(e.h, ptr(out))
+    assert out[0] > 0 and out[1] == 0 and out[2] == 0
