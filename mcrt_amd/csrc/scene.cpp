@@ -426,6 +426,9 @@ int finalize_scene(mcrt_scene* s, int threads, const char* cache)
         if (!device_records(wb, dn))
             return fail(MCRT_ERR_OUT_OF_MEMORY, "BVH of %zu nodes and %zu references exceeds 2^29 records",
                         wb.qnodes.size(), wb.refs.size());
+        // a scene without nodes gets one without children: the kernels start
+        // at record 0 unconditionally
+        if (dn.empty()) dn.push_back(quantize_node(empty_node()));
         const size_t nb = dn.size() * sizeof(QNode), rb = wb.refs.size() * sizeof(WRef);
         if ((rc = s->d_bvh.ensure(nb + rb))) return rc;
         hipError_t e = hipSuccess;
@@ -441,7 +444,7 @@ int finalize_scene(mcrt_scene* s, int threads, const char* cache)
     if ((rc = upload_materials(s))) return rc;
 
     DevScene& d = s->dev;
-    d.nodes = wb.qnodes.empty() ? nullptr : s->d_bvh.as<QNode>();
+    d.nodes = s->d_bvh.as<QNode>();
     d.shade = s->d_shade.as<TriShade>();
     d.verts = s->d_verts.as<float>();
     d.lights = s->d_lights.as<DevLight>();

@@ -360,8 +360,15 @@ bool device_records(const WideBVH& wb, std::vector<QNode>& nodes_out)
     return true;
 }
 
-namespace
+WNode empty_node()
 {
+    WNode w;
+    std::memset(&w, 0, sizeof(w));
+    for (int s = 0; s < 4; s++) w.child[s] = MCRT_CHILD_EMPTY;
+    w.order_lo = w.order_hi = 0xe4e4e4e4u;  // slot order in every octant
+    return w;
+}
+
 QNode quantize_node(const WNode& w)
 {
     QNode q;
@@ -390,7 +397,6 @@ QNode quantize_node(const WNode& w)
     q.rank_hi = order_to_rank(w.order_hi);
     return q;
 }
-}  // namespace
 
 void quantize_nodes(WideBVH& out)
 {

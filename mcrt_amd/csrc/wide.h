@@ -18,6 +18,10 @@ struct WideBVH
 
 void collapse_wide(const BTree& bt, const std::vector<Tri>& tris, WideBVH& out);
 
+// A node without children, and a node quantised for the kernels.
+WNode empty_node();
+QNode quantize_node(const WNode& w);
+
 // Fills out.qnodes from out.nodes (collapse_wide calls it).
 void quantize_nodes(WideBVH& out);
 

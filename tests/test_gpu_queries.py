@@ -279,3 +279,23 @@ def test_fixed_windows_and_claims_bit_exact(ctx, n):
         assert np.array_equal(prim, want[0])
         assert np.array_equal(tuv.view(np.uint32), want[1].view(np.uint32))
         assert np.array_equal(s.occluded(rays, np.full(n, 7, np.uint8)), (want[0] >= 0).astype(np.uint8))
+
+
+def test_special_rays_and_empty_scene(ctx):
+    """Zero, tiny, infinite and NaN components and limits against the oracle;
+    a scene without triangles misses every ray."""
+    import mcrt_amd
+    from test_product_host import special_rays
+    tris = _libs.debug_mesh()
+    s, _ = _scene(ctx, tris)
+    rays = special_rays(tris)
+    op, otuv = _libs.OracleBVH(tris).intersect(rays)
+    prim, tuv = mcrt_amd.split_hits(s.intersect(rays))
+    assert np.array_equal(prim, op)
+    assert np.array_equal(tuv.view(np.uint32), otuv.view(np.uint32))
+    assert np.array_equal(s.occluded(rays), (op >= 0).astype(np.uint8))
+    e = mcrt_amd.Scene(ctx)
+    e.finalize()
+    prim, tuv = mcrt_amd.split_hits(e.intersect(rays))
+    assert (prim == -1).all() and np.isposinf(tuv[:, 0]).all() and (tuv[:, 1:] == 0).all()
+    assert (e.occluded(rays) == 0).all()

@@ -269,3 +269,45 @@ def test_optimised_nodes_keep_every_hit(emu, which):
     out = np.zeros(4, np.int64)
     e.L.emu_check_qnodes(e.h, ptr(out))
     assert out[0] > 0 and out[1] == 0 and out[2] == 0
+
+
+def special_rays(tris, n=4096, seed=9):
+    """Rays through the mesh with one thing wrong or extreme each: zero, tiny,
+    infinite and NaN direction components, infinite and NaN origins, tmin
+    above tmax, NaN, infinite and negative limits, all-zero directions."""
+    r = _libs.random_rays(tris, n, seed=seed)
+    rng = np.random.default_rng(seed)
+    nan, inf = np.float32(np.nan), np.float32(np.inf)
+    for i in range(n):
+        k, a = i % 14, int(rng.integers(3))
+        if k == 0: r[i, 4 + a] = 0.0
+        elif k == 1: r[i, 4 + a] = np.float32(1e-42) * rng.choice([-1, 1])
+        elif k == 2: r[i, 4:7] = 0.0
+        elif k == 3: r[i, 4 + a] = nan
+        elif k == 4: r[i, a] = nan
+        elif k == 5: r[i, a] = inf * rng.choice([-1, 1])
+        elif k == 6: r[i, 4 + a] = inf
+        elif k == 7: r[i, 3], r[i, 7] = 2.0, 1.0
+        elif k == 8: r[i, 3] = nan
+        elif k == 9: r[i, 7] = nan
+        elif k == 10: r[i, 3], r[i, 7] = -inf, inf
+        elif k == 11: r[i, 4:7] *= np.float32(1e-38)
+        elif k == 12: r[i, 4:7] *= np.float32(1e30)
+    return r
+
+
+@pytest.mark.parametrize("which", ["debug_mesh", "soup_slice"])
+def test_special_rays_equal_oracle(emu, which):
+    """Rays outside the ordinary range (special_rays) give the oracle's hits
+    through the conservative node tests, whose exact rays and non-finite
+    origins are constants of the plane map."""
+    tris = _libs.debug_mesh() if which == "debug_mesh" else _libs.soup_slice()
+    rays = special_rays(tris)
+    e = Emu(tris)
+    e.L.emu_optimize(e.h, ptr(np.zeros(8, np.int64)))
+    prim, tuv = _libs.OracleBVH(tris).intersect(rays)
+    hits, _ = e.trace(rays)
+    assert np.array_equal(hits[:, 0], prim)
+    assert np.array_equal(hits[:, 1:].view(np.uint32), tuv.view(np.uint32))
+    occ, _ = e.trace(rays, any_hit=True)
+    assert np.array_equal(occ, (prim >= 0).astype(np.uint8))
