@@ -277,17 +277,23 @@ __device__ __forceinline__ void grad_add(float* acc, float* g, int key, int hot,
     scatter3(g, key, v, valid && hot < 0);
 }
 
-// Counts of one side, and its traversal work counters zeroed.
+// The counts of one side set and its traversal work counters zeroed, by the
+// first workgroup of a kernel that runs before the side's next use: k_generate
+// sets both sides, k_resolve of vertex k clears the side that k_shade of
+// vertex k fills (last read by the shade of vertex k - 1).  Launches of their
+// own for this, and a resolve of the first vertex, which has no records, cost
+// a 97x61 one-sample frame 18 us (543 -> 525 us).
 constexpr int kCntWq = 64;
 static_assert(kSeg2Word >= 32 && kSeg2Word < kCntWq, "the third count sits on its own 128 B line before the work counters");
 constexpr int kSideWords = kCntWq + (int)kWqWords;
-__global__ void k_set_counts(uint32_t* cnt, uint32_t a, uint32_t b)
+__device__ __forceinline__ void set_counts(uint32_t* cnt, uint32_t a)
 {
-    if (blockIdx.x == 0 && threadIdx.x < kSlices) cnt[kCntWq + threadIdx.x * kSliceStride] = 0;
-    if (threadIdx.x == 0 && blockIdx.x == 0)
+    if (blockIdx.x != 0) return;
+    if (threadIdx.x < kSlices) cnt[kCntWq + threadIdx.x * kSliceStride] = 0;
+    if (threadIdx.x == 0)
     {
         cnt[0] = a;
-        cnt[1] = b;
+        cnt[1] = 0;
         cnt[kSeg2Word] = 0;
     }
 }
@@ -319,6 +325,8 @@ __device__ __forceinline__ int find_seg(const Segment* seg, int nseg, int64_t x)
 template <bool BATCH>
 __global__ void k_generate(PTState S, PTArgs a)
 {
+    set_counts(S.cnt[0], (uint32_t)a.P);
+    set_counts(S.cnt[1], 0u);
     for (int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; p < a.P; p += (int64_t)gridDim.x * blockDim.x)
     {
         const ScenePT* sp = &a.one;
@@ -445,6 +453,7 @@ __global__ void k_resolve(PTArgs a, PTState S, int cur)
 {
     __shared__ float acc[ADJ ? 2 * kHotFloats : 1];
     if (ADJ) hot_clear(acc);
+    set_counts(S.cnt[cur ^ 1], 0u);
     const int64_t P = a.P;
     constexpr int rs = ENV ? 4 : 2, rf = rec_rays(rs);
     const uint32_t nrec = S.cnt[cur][1] / (uint32_t)rf;
@@ -910,18 +919,20 @@ template <bool ADJ, bool BATCH>
 void bounce_loop(const DevScene& Dt, PTState& S, const PTArgs& a, int max_depth, int cus, hipStream_t st)
 {
     hipLaunchKernelGGL(k_generate<BATCH>, (grid_of<k_generate<BATCH>>(a.P, cus)), dim3(kTPB), 0, st, S, a);
-    hipLaunchKernelGGL(k_set_counts, dim3(1), dim3(64), 0, st, S.cnt[0], (uint32_t)a.P, 0u);
     int cur = 0;
     for (int k = 0; k <= max_depth + 1; k++)
     {
-        const int nxt = cur ^ 1;
         TraceBatch tb;
         tb.roots = a.roots;
         tb.rsid = S.rsid[cur];
         launch_k_trace<false, false, true, BATCH>(Dt, trace_blocks(Dt, (1 + a.rs) * a.P), st, S.rays[cur], (int64_t)0,
                                                   S.cnt[cur], a.P, a.P + rec_rays(a.rs) * a.P, S.hits, (uint8_t*)nullptr,
                                                   (unsigned long long*)nullptr, S.cnt[cur] + kCntWq, tb);
-        if (a.rs == 4)
+        if (k == 0)
+        {
+            // no records yet
+        }
+        else if (a.rs == 4)
             hipLaunchKernelGGL((k_resolve<ADJ, BATCH, true>), (grid_of<k_resolve<ADJ, BATCH, true>>(a.P, cus)),
                                dim3(kTPB), 0, st, a, S, cur);
         else
@@ -929,7 +940,6 @@ void bounce_loop(const DevScene& Dt, PTState& S, const PTArgs& a, int max_depth,
                                dim3(kTPB), 0, st, a, S, cur);
         if (k <= max_depth)
         {
-            hipLaunchKernelGGL(k_set_counts, dim3(1), dim3(64), 0, st, S.cnt[nxt], 0u, 0u);
             if (a.rs == 4)
                 hipLaunchKernelGGL((k_shade<ADJ, BATCH, true>), (grid_of<k_shade<ADJ, BATCH, true>>(a.P, cus)),
                                    dim3(kTPB), 0, st, a, S, cur, k);
@@ -937,7 +947,7 @@ void bounce_loop(const DevScene& Dt, PTState& S, const PTArgs& a, int max_depth,
                 hipLaunchKernelGGL((k_shade<ADJ, BATCH, false>), (grid_of<k_shade<ADJ, BATCH, false>>(a.P, cus)),
                                    dim3(kTPB), 0, st, a, S, cur, k);
         }
-        cur = nxt;
+        cur ^= 1;
     }
 }
 
