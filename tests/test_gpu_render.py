@@ -217,3 +217,36 @@ def test_render_errors(ctx):
     with pytest.raises(mcrt_amd.McrtError) as e:
         s.render(spp=(1 << 28) + 1)  # one pixel's samples must fit a wavefront chunk
     assert e.value.code == 1 and b"spp" in mcrt_amd.lib().mcrt_last_error()
+
+
+@pytest.mark.parametrize("what", ["black", "negative", "inf albedo", "nan albedo", "inf light", "dark light",
+                                  "negative light", "odd light normals"])
+def test_render_bit_exact_extreme_terms(ctx, what):
+    """Next-event terms that are zero, negative, infinite or NaN in the light
+    or in the dark, and light normals that face away over part of the light:
+    a shadow ray left out or a term formed before its visibility is known
+    must not change a bit of the film."""
+    from mcrt_amd import scenes
+    d = scenes.cornell_icosphere(2)
+    rgb, normals = d.mat_rgb.copy(), d.normals.copy().reshape(-1, 3, 3)
+    if what == "black":
+        rgb[4] = 0.0
+    elif what == "negative":
+        rgb[4] = (-0.5, 0.8, 0.0)
+    elif what == "inf albedo":
+        rgb[4] = (np.inf, 0.5, 0.0)
+    elif what == "nan albedo":
+        rgb[4] = (0.5, np.nan, 0.5)
+    elif what == "inf light":
+        rgb[0] = (np.inf, 15.0, 0.0)
+    elif what == "dark light":
+        rgb[0] = 0.0
+    elif what == "negative light":
+        rgb[0] = (-15.0, 15.0, 15.0)
+    else:
+        normals[0, 0] = (0.0, 1.0, 0.0)   # one corner of the light turned up
+        normals[1, 2] = (1.0, 0.1, 0.0)
+    d = scenes.SceneData(d.tris, normals, d.tri_mat, d.mat_type, rgb, d.mat_gloss)
+    kw = dict(spp=4, max_depth=4, rr_start=2, rr_prob=0.8, seed=3, nee=True)
+    print(f"[extreme terms: {what}]", flush=True)
+    _compare(what, gpu_render(ctx, d, 40, 33, **kw), oracle_render(d, 40, 33, **kw))
