@@ -69,10 +69,11 @@ struct PTState
                          //  P BSDF-sampled next-event, compacted] x 2 float4 per ray
     uint32_t* act[2];    // path id per continuation ray
     float4* rec[2];      // next-event records, rec_words(rs) float4 each
-    float4* sh[2];       // forward, no environment map: per light-sample shadow ray the
+    float4* sh[2];       // no environment map: per light-sample shadow ray the
                          // radiance {x, y, z} it adds to path w where it reaches its
                          // light (w = ~0: the vertex has a record, which adds it)
     uint32_t* want[2];   // and the light triangle it must hit
+    float4* shg[2];      // adjoint: and that triangle's emission gradient, its hot slot in w
     uint32_t* bsl[2];    // with an environment map: each record's BSDF-sampled ray slot or ~0
                          // (its 64 B record has no spare word)
     uint32_t* cnt[2];    // {continuation rays, next-event rays at record slots}, the
@@ -831,8 +832,7 @@ __global__ void k_shade(PTArgs a, PTState S, int cur, int k)
     if (ADJ) hot_flush(a.one.D, acc, S.g_alb, S.g_em);
 }
 
-// One vertex of every live path in a forward render without an environment
-// map.  The light sample comes before the workgroup takes its slots, with the
+// One vertex of every live path in a render without an environment map.  The light sample comes before the workgroup takes its slots, with the
 // sampled triangle's own Moller-Trumbore test (the traversal's arithmetic on
 // the traversal's operands, so its t, u, v are those of a hit): a shadow ray
 // exists only where its triangle can be hit, faces the vertex and adds
@@ -848,9 +848,11 @@ __global__ void k_shade(PTArgs a, PTState S, int cur, int k)
 // term), next-event sums 8.3 -> 4.2 ms, this kernel 15.2 -> 14.8 ms at 76
 // instead of 86 registers (6 waves per SIMD).  Bound by the latency of its
 // dependent loads (path, hit, triangle, material) and by its stores.
-template <bool BATCH>
+template <bool ADJ, bool BATCH>
 __global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
 {
+    __shared__ float acc[ADJ ? 2 * kHotFloats : 1];
+    if (ADJ) hot_clear(acc);
     const int nxt = cur ^ 1;
     const uint32_t A = S.cnt[cur][0];
     const float4* rays = S.rays[cur];
@@ -901,9 +903,9 @@ __global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
             no_direct = !sp.nee || t4.w == 0.0f;
         }
         const V3f col = ld3(mt.rgb);
-        V3f wo = zero, x = zero;
+        V3f wo = zero, x = zero, c2 = zero;
         float factor2 = 0.0f;
-        int li = -1, tri = -1;
+        int li = -1, tri = -1, tri_hot = -1;
         bool want_sh = false;
         if (want_rec)
         {
@@ -922,11 +924,13 @@ __global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
                 r.ox = phit.x; r.oy = phit.y; r.oz = phit.z;
                 r.dx = wo.x; r.dy = wo.y; r.dz = wo.z;
                 float t, u, v;
-                if (mcrt::mt(r, v0.x, v0.y, v0.z, e1.x, e1.y, e1.z, e2.x, e2.y, e2.z, D.det_eps, t, u, v) && t > kEpsRay && t < __builtin_inff())
+                if (mcrt::mt(r, v0.x, v0.y, v0.z, e1.x, e1.y, e1.z, e2.x, e2.y, e2.z, D.det_eps, t, u, v) &&
+                    t > kEpsRay && t < __builtin_inff())
                 {
                     const TriShade tl = D.shade[tri];
                     reach = !(dot(shading_normal(tl, u, v), -wo) < 0);
                     le = ld3(D.mats[tl.mat].rgb);
+                    tri_hot = tl.hot;
                 }
             }
             // area_terms with a missing BSDF-sampled ray, the light visible and not
@@ -935,24 +939,45 @@ __global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
             const V3f f = v3f(ip, ip, ip) * col;
             const V3f lit = (f * le) * factor2, dark = (f * zero) * factor2;
             want_sh = reach && !(lit.x == dark.x && lit.y == dark.y && lit.z == dark.z);
+            if (ADJ)  // the coefficient of the emission counts where the emission is zero, too
+            {
+                c2 = f * factor2;
+                want_sh = want_sh || (reach && !(c2.x == 0.0f && c2.y == 0.0f && c2.z == 0.0f));
+            }
             x = T * (none + lit);
             const V3f x0 = T * (li >= 0 ? none + dark : none);
             // a term that is not zero in the dark (infinite or NaN colours or
             // throughput) is left to a record
             if (!(x0.x == 0.0f && x0.y == 0.0f && x0.z == 0.0f)) trace_wb = true;
-            if (!trace_wb && x.x == 0.0f && x.y == 0.0f && x.z == 0.0f) want_sh = false;
+            if (!ADJ && !trace_wb && x.x == 0.0f && x.y == 0.0f && x.z == 0.0f) want_sh = false;
         }
         uint32_t cslot, sslot, bslot;
         block_slots(S.cnt[nxt], want_cont, want_sh, trace_wb, 1u, cslot, sslot, bslot);
-        if (!hit) continue;
-        if (mt.type == MCRT_LGHT)
+        int alb_key = -1, em_key = -1, hot = -1;
+        V3f g_alb = zero, g_em = zero;
+        if (hit && mt.type == MCRT_LGHT)
         {
             if (no_direct && dot(d, ns) < 0)
             {
                 const V3f Lv = f3(S.L[p]) + T * col;
                 S.L[p] = f4(Lv);
+                if (ADJ)
+                {
+                    em_key = h.x;
+                    hot = ts.hot;
+                    g_em = f3(S.delta[p]) * T;
+                }
             }
-            continue;
+        }
+        else if (ADJ && hit)
+        {
+            // every later term carries this vertex's albedo once
+            const V3f rest = f3(S.Ltot[p]) - f3(S.L[p]);
+            const V3f dl = f3(S.delta[p]);
+            alb_key = h.x;
+            hot = ts.hot;
+            g_alb = v3f(col.x > 0.0f ? dl.x * rest.x / col.x : 0.0f, col.y > 0.0f ? dl.y * rest.y / col.y : 0.0f,
+                        col.z > 0.0f ? dl.z * rest.z / col.z : 0.0f);
         }
         float4* nr = S.rays[nxt];
         if (want_sh)
@@ -961,6 +986,11 @@ __global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
             store_ray(nr, r1, phit, wo, kEpsRay, __builtin_inff());
             S.sh[nxt][sslot] = make_float4(x.x, x.y, x.z, float_of(trace_wb ? ~0u : p));
             S.want[nxt][sslot] = (uint32_t)tri;
+            if (ADJ)
+            {
+                const V3f g = (f3(S.delta[p]) * T) * c2;
+                S.shg[nxt][sslot] = make_float4(g.x, g.y, g.z, float_of((uint32_t)tri_hot));
+            }
             if (BATCH) S.rsid[nxt][r1] = sid;
         }
         if (trace_wb)
@@ -973,63 +1003,110 @@ __global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
             store_ray(nr, r2, phit, wb, kEpsRay, __builtin_inff());
             if (BATCH) S.rsid[nxt][r2] = sid;
         }
-        if (!want_cont) continue;
-        // Continuation (Material::sample, demo_pt.cpp:645-650)
-        const V3f wi = -d;
-        V3f nd, weight;
-        if (mt.type == MCRT_GLSY)
+        if (want_cont)
         {
-            float w;
-            nd = glossy_dir(wi, ns, mt.gloss, rng_u01(key, 5), rng_u01(key, 6), w);
-            weight = col * w;
+            // Continuation (Material::sample, demo_pt.cpp:645-650)
+            const V3f wi = -d;
+            V3f nd, weight;
+            if (mt.type == MCRT_GLSY)
+            {
+                float w;
+                nd = glossy_dir(wi, ns, mt.gloss, rng_u01(key, 5), rng_u01(key, 6), w);
+                weight = col * w;
+            }
+            else
+            {
+                nd = lambert_dir(ns, rng_u01(key, 5), rng_u01(key, 6));
+                weight = col;
+            }
+            T = T * weight;
+            if (k >= sp.rr_start) T = T * (1.0f / sp.rr_prob);
+            S.T[p] = make_float4(T.x, T.y, T.z, mt.type == MCRT_DIFF ? 1.0f : 0.0f);
+            store_ray(nr, cslot, phit, nd, kEpsRay, __builtin_inff());
+            S.act[nxt][cslot] = p;
+            if (BATCH) S.rsid[nxt][cslot] = sid;
         }
-        else
+        if (ADJ)
         {
-            nd = lambert_dir(ns, rng_u01(key, 5), rng_u01(key, 6));
-            weight = col;
+            grad_add(acc, S.g_alb, alb_key, hot, g_alb, alb_key >= 0);
+            grad_add(acc + kHotFloats, S.g_em, em_key, hot, g_em, em_key >= 0);
         }
-        T = T * weight;
-        if (k >= sp.rr_start) T = T * (1.0f / sp.rr_prob);
-        S.T[p] = make_float4(T.x, T.y, T.z, mt.type == MCRT_DIFF ? 1.0f : 0.0f);
-        store_ray(nr, cslot, phit, nd, kEpsRay, __builtin_inff());
-        S.act[nxt][cslot] = p;
-        if (BATCH) S.rsid[nxt][cslot] = sid;
     }
+    if (ADJ) hot_flush(a.one.D, acc, S.g_alb, S.g_em);
 }
 
 // The next-event terms k_shade_direct left: a shadow ray whose closest hit is
 // its light's triangle adds its term, then the records of the BSDF-sampled
 // rays.  A vertex has one or the other, so no two threads add to one path.
-template <bool BATCH>
+template <bool ADJ, bool BATCH>
 __global__ void k_direct(PTArgs a, PTState S, int cur)
 {
+    __shared__ float acc[ADJ ? 2 * kHotFloats : 1];
+    if (ADJ) hot_clear(acc);
     set_counts(S.cnt[cur ^ 1], 0u);
-    const uint32_t nsh = S.cnt[cur][1], nrec = S.cnt[cur][kSeg2Word];
-    const int64_t first = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t s = first; s < nsh; s += step)
+    const int64_t nsh = S.cnt[cur][1], nrec = S.cnt[cur][kSeg2Word];
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+    // every lane runs every iteration of its wave: the gradient sums need them all
+    for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < nsh; base += step)
     {
-        const float4 xp = S.sh[cur][s];
-        const uint32_t path = bits_of(xp.w);
-        if (path != ~0u && S.hits[a.P + s].x == (int)S.want[cur][s]) S.L[path] = f4(f3(S.L[path]) + f3(xp));
+        const int64_t s = base + threadIdx.x;
+        int em = -1, hot = -1;
+        V3f g = v3f(0.0f, 0.0f, 0.0f);
+        if (s < nsh)
+        {
+            const float4 xp = S.sh[cur][s];
+            const uint32_t path = bits_of(xp.w);
+            const int tri = (int)S.want[cur][s];
+            if (path != ~0u && S.hits[a.P + s].x == tri)
+            {
+                const V3f x = f3(xp);
+                // a zero term leaves the path's radiance as it is (k_resolve)
+                if (!ADJ || !(x.x == 0.0f && x.y == 0.0f && x.z == 0.0f)) S.L[path] = f4(f3(S.L[path]) + x);
+                if (ADJ)
+                {
+                    const float4 gh = S.shg[cur][s];
+                    em = tri;
+                    hot = (int)bits_of(gh.w);
+                    g = f3(gh);
+                }
+            }
+        }
+        if (ADJ) grad_add(acc + kHotFloats, S.g_em, em, hot, g, em >= 0);
     }
     const float4* rays = S.rays[cur];
-    for (int64_t m = first; m < nrec; m += step)
+    for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < nrec; base += step)
     {
-        const float4* Rm = S.rec[cur] + rec_words(2) * m;
-        const float4 r0 = Rm[0], r1 = Rm[1], r2 = Rm[2];
-        const uint32_t path = bits_of(r2.x);
-        const int li = (int)bits_of(r2.y), ss = (int)bits_of(r2.z);
-        const DevScene& D = BATCH ? a.tab[S.sid[path]].D : a.one.D;
-        const int64_t hb = 2 * a.P + m, hs = a.P + ss;
-        int em1, em2, hot1, hot2;
-        V3f c1, c2;
-        const V3f local = area_terms(D, S.hits[hb], ss >= 0 ? S.hits[hs] : make_int4(-1, 0, 0, 0), f3(r1),
-                                     rays + 2 * hb, rays + 2 * hs, r0.w, r1.w, li, v3f(0.0f, 0.0f, 0.0f), em1, em2,
-                                     hot1, hot2, c1, c2);
-        // zero terms leave the path's radiance as it is (k_resolve)
-        const V3f x = f3(r0) * local;
-        if (!(x.x == 0.0f && x.y == 0.0f && x.z == 0.0f)) S.L[path] = f4(f3(S.L[path]) + x);
+        const int64_t m = base + threadIdx.x;
+        int em1 = -1, em2 = -1, hot1 = -1, hot2 = -1;
+        V3f g1 = v3f(0.0f, 0.0f, 0.0f), g2 = g1;
+        if (m < nrec)
+        {
+            const float4* Rm = S.rec[cur] + rec_words(2) * m;
+            const float4 r0 = Rm[0], r1 = Rm[1], r2 = Rm[2];
+            const uint32_t path = bits_of(r2.x);
+            const int li = (int)bits_of(r2.y), ss = (int)bits_of(r2.z);
+            const DevScene& D = BATCH ? a.tab[S.sid[path]].D : a.one.D;
+            const int64_t hb = 2 * a.P + m, hs = a.P + ss;
+            V3f c1, c2;
+            const V3f local = area_terms(D, S.hits[hb], ss >= 0 ? S.hits[hs] : make_int4(-1, 0, 0, 0), f3(r1),
+                                         rays + 2 * hb, rays + 2 * hs, r0.w, r1.w, li, v3f(0.0f, 0.0f, 0.0f), em1,
+                                         em2, hot1, hot2, c1, c2);
+            const V3f T = f3(r0), x = T * local;
+            if (!(x.x == 0.0f && x.y == 0.0f && x.z == 0.0f)) S.L[path] = f4(f3(S.L[path]) + x);
+            if (ADJ)
+            {
+                const V3f dl = f3(S.delta[path]);
+                g1 = (dl * T) * c1;
+                g2 = (dl * T) * c2;
+            }
+        }
+        if (ADJ)
+        {
+            grad_add(acc + kHotFloats, S.g_em, em1, hot1, g1, em1 >= 0);
+            grad_add(acc + kHotFloats, S.g_em, em2, hot2, g2, em2 >= 0);
+        }
     }
+    if (ADJ) hot_flush(a.one.D, acc, S.g_alb, S.g_em);
 }
 
 // Adjoint seed: keep pass 1's radiance and form dLoss/dL of each path
@@ -1160,22 +1237,17 @@ void bounce_loop(const DevScene& Dt, PTState& S, const PTArgs& a, int max_depth,
         else if (a.rs == 4)
             hipLaunchKernelGGL((k_resolve<ADJ, BATCH, true>), (grid_of<k_resolve<ADJ, BATCH, true>>(a.P, cus)),
                                dim3(kTPB), 0, st, a, S, cur);
-        else if constexpr (ADJ)
-            hipLaunchKernelGGL((k_resolve<true, BATCH, false>), (grid_of<k_resolve<true, BATCH, false>>(a.P, cus)),
-                               dim3(kTPB), 0, st, a, S, cur);
         else
-            hipLaunchKernelGGL(k_direct<BATCH>, (grid_of<k_direct<BATCH>>(a.P, cus)), dim3(kTPB), 0, st, a, S, cur);
+            hipLaunchKernelGGL((k_direct<ADJ, BATCH>), (grid_of<k_direct<ADJ, BATCH>>(a.P, cus)), dim3(kTPB), 0, st, a,
+                               S, cur);
         if (k <= max_depth)
         {
             if (a.rs == 4)
                 hipLaunchKernelGGL((k_shade<ADJ, BATCH, true>), (grid_of<k_shade<ADJ, BATCH, true>>(a.P, cus)),
                                    dim3(kTPB), 0, st, a, S, cur, k);
-            else if constexpr (ADJ)
-                hipLaunchKernelGGL((k_shade<true, BATCH, false>), (grid_of<k_shade<true, BATCH, false>>(a.P, cus)),
-                                   dim3(kTPB), 0, st, a, S, cur, k);
             else
-                hipLaunchKernelGGL(k_shade_direct<BATCH>, (grid_of<k_shade_direct<BATCH>>(a.P, cus)), dim3(kTPB), 0,
-                                   st, a, S, cur, k);
+                hipLaunchKernelGGL((k_shade_direct<ADJ, BATCH>), (grid_of<k_shade_direct<ADJ, BATCH>>(a.P, cus)),
+                                   dim3(kTPB), 0, st, a, S, cur, k);
         }
         cur ^= 1;
     }
@@ -1194,9 +1266,10 @@ PTState state_of(StreamRes* r, int64_t P, bool adjoint)
         S.act[i] = w.act[i].as<uint32_t>();
         S.rec[i] = w.rec[i].as<float4>();
         S.bsl[i] = w.bsl[i].as<uint32_t>();
-        // a forward render's shadow-ray terms follow its P records (pt_workspace)
+        // the shadow rays' terms follow the P records (pt_workspace)
         S.sh[i] = S.rec[i] + rec_words(2) * P;
-        S.want[i] = reinterpret_cast<uint32_t*>(S.sh[i] + P);
+        S.shg[i] = S.sh[i] + P;
+        S.want[i] = reinterpret_cast<uint32_t*>(S.shg[i] + (adjoint ? P : 0));
         S.cnt[i] = w.cnt.as<uint32_t>() + kSideWords * i;
         S.rsid[i] = w.rsid[i].as<uint16_t>();
     }
@@ -1242,7 +1315,8 @@ int pt_workspace(StreamRes* r, int64_t P, bool adjoint, bool batch, int rs)
         if ((rc = w.rays[i].ensure(nr * 32))) return rc;
         if ((rc = w.act[i].ensure(n * 4))) return rc;
         // without an environment map also the shadow rays' terms and triangles
-        if ((rc = w.rec[i].ensure(n * (16 * rec_words(rs) + (rs == 4 ? 0 : 20))))) return rc;
+        // (and, for the adjoint, gradients)
+        if ((rc = w.rec[i].ensure(n * (16 * rec_words(rs) + (rs == 4 ? 0 : adjoint ? 36 : 20))))) return rc;
         if (rs == 4 && (rc = w.bsl[i].ensure(n * 4))) return rc;
     }
     if ((rc = w.cnt.ensure(2 * kSideWords * sizeof(uint32_t)))) return rc;
