@@ -39,6 +39,7 @@ struct DevScene
     const DevMaterial* mats = nullptr;
     const DevLight* lights = nullptr;
     int32_t nlights = 0;
+    bool big = false;                  // the BVH takes kBigBvhBytes or more
     int32_t stack_bound = 0;
     const int32_t* hot_tri = nullptr;  // triangle of each gradient hot slot
     int32_t nhot = 0;
@@ -92,6 +93,9 @@ struct SceneRoot
 // any hit 7 (held to eight waves' registers it spills scalar registers).
 constexpr int kTraceWavesPerSimd = 8;
 constexpr int kTraceAnyWavesPerSimd = 7;
+
+// Below this the kernels form a BVH record's byte offset in 32 bits.
+constexpr size_t kBigBvhBytes = size_t(1) << 32;
 
 // Work counters of a traversal launch: one per slice of the rays, 64 B
 // apart (trace_kernel.h).

@@ -1465,6 +1465,7 @@ int batch_init(mcrt_batch* b)
     Dt = s0->dev;
     Dt.nodes = nullptr;
     Dt.stack_bound = max_sb;
+    for (const mcrt_scene* s : b->scenes) Dt.big = Dt.big || s->dev.big;
     trace_geometry(Dt, b->ctx->num_cus, s0->pt_trace_waves_per_cu, s0->pt_trace_lds_depth);
     Dt.refill_lanes = s0->pt_trace_refill_lanes;
     if (Dt.spill_depth > 0)

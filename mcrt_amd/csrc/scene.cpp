@@ -421,14 +421,14 @@ int finalize_scene(mcrt_scene* s, int threads, const char* cache)
 
     int rc;
     {
-        // one array of 64 B records, nodes then references (layout.h)
+        // one array of 64 B records, nodes then references (layout.h); a
+        // scene without nodes gets one without children, since the kernels
+        // start at record 0 unconditionally
+        if (wb.qnodes.empty()) wb.qnodes.push_back(quantize_node(empty_node()));
         std::vector<QNode> dn;
         if (!device_records(wb, dn))
             return fail(MCRT_ERR_OUT_OF_MEMORY, "BVH of %zu nodes and %zu references exceeds 2^29 records",
                         wb.qnodes.size(), wb.refs.size());
-        // a scene without nodes gets one without children: the kernels start
-        // at record 0 unconditionally
-        if (dn.empty()) dn.push_back(quantize_node(empty_node()));
         const size_t nb = dn.size() * sizeof(QNode), rb = wb.refs.size() * sizeof(WRef);
         if ((rc = s->d_bvh.ensure(nb + rb))) return rc;
         hipError_t e = hipSuccess;
@@ -445,6 +445,7 @@ int finalize_scene(mcrt_scene* s, int threads, const char* cache)
 
     DevScene& d = s->dev;
     d.nodes = s->d_bvh.as<QNode>();
+    d.big = s->d_bvh.bytes >= kBigBvhBytes;
     d.shade = s->d_shade.as<TriShade>();
     d.verts = s->d_verts.as<float>();
     d.lights = s->d_lights.as<DevLight>();
@@ -625,7 +626,8 @@ int read_envmap(const char* path, int& w, int& h, std::vector<float>& rgb)
 
 void trace_geometry(DevScene& d, int num_cus, int waves_per_cu, int lds_depth)
 {
-    d.lds_depth = lds_depth;
+    // the kernels for BVHs of 4 GB and more exist with the smallest LDS stack
+    d.lds_depth = d.big ? 8 : lds_depth;
     d.spill_lanes = (int64_t)num_cus * waves_per_cu * 64;
     const int any_waves = 4 * kTraceAnyWavesPerSimd;
     d.lanes_any = (int64_t)num_cus * (waves_per_cu < any_waves ? waves_per_cu : any_waves) * 64;

@@ -177,12 +177,13 @@ MCRT_HD void node_margin(RayPrep& r, float span)
 // plane words already ordered near / far per axis by the ray's signs, and
 // per axis the plane map's slope s * inv (a*) and its lower / upper offsets
 // (n*, f*).
-MCRT_HD bool qslab_c(const RayPrep& r, uint32_t child, uint32_t nx, uint32_t fx, uint32_t ny, uint32_t fy,
+MCRT_HD bool qslab_c(const RayPrep& r, uint32_t nx, uint32_t fx, uint32_t ny, uint32_t fy,
                      uint32_t nz, uint32_t fz, float ax, float ay, float az, float nbx, float fbx, float nby,
                      float fby, float nbz, float fbz, int shift, float R1, float& lo)
 {
-    // computed for every slot (an empty slot's planes decode to finite
-    // values), so the four tests need no branches
+    // computed for every slot: an empty slot's planes are inverted, and its
+    // link leads to a reference that nothing hits, should a node be so small
+    // against the margin that they pass (device_records, wide.cpp)
     const float t0x = __builtin_fmaf((float)((nx >> shift) & 0xffu), ax, nbx);
     const float t1x = __builtin_fmaf((float)((fx >> shift) & 0xffu), ax, fbx);
     const float t0y = __builtin_fmaf((float)((ny >> shift) & 0xffu), ay, nby);
@@ -193,7 +194,7 @@ MCRT_HD bool qslab_c(const RayPrep& r, uint32_t child, uint32_t nx, uint32_t fx,
     // adds, R0 <= R1, fails only where no hit can be accepted
     lo = fmaxf(fmaxf(fmaxf(t0x, t0y), t0z), r.R0);
     const float hi = fminf(fminf(fminf(t1x, t1y), t1z), R1);
-    return (lo <= hi) & (child != MCRT_CHILD_EMPTY);
+    return lo <= hi;
 }
 
 // rayTriangleIntersect (triangle.cpp:13-51), e1/e2 precomputed; `eps` is
@@ -290,7 +291,8 @@ struct TraceCount
 // The traversal of one ray as a sequence of steps (one wide node or one
 // leaf per step), so a kernel can hand a lane its next ray as soon as the
 // current one ends instead of waiting for the wavefront's slowest lane.
-template <bool ANY, bool COUNT>
+// BIG: the record array may hold 2^26 records or more (record()).
+template <bool ANY, bool COUNT, bool BIG>
 struct Tracer
 {
     RayPrep r;
@@ -311,10 +313,16 @@ struct Tracer
 
     // The 64 B record `cur` names: a QNode, or a leaf reference, both in the
     // scene's one record array (layout.h).  Sc is any type with the scene's
-    // `nodes` and `det_eps` (DevScene, SceneRoot).
+    // `nodes` and `det_eps` (DevScene, SceneRoot).  With fewer than 2^26
+    // records (!BIG) the record's 32-bit byte offset is one shift, which also
+    // drops a leaf link's flag and count, and the loads take the array's
+    // address from scalar registers: 16M rays of the 1.3M-triangle mesh 1,409
+    // -> 1,356 us, 8M of the 2M-triangle soup 3,622 -> 3,378, against 64-bit
+    // addresses formed per lane.
     template <class Sc>
     MCRT_HD const uint4* record(const Sc& S) const
     {
+        if (!BIG) return reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(S.nodes) + (uint32_t)(cur << 6));
         return reinterpret_cast<const uint4*>(S.nodes) + 4 * (size_t)(cur & MCRT_LEAF_REF_MASK);
     }
 
@@ -353,10 +361,10 @@ struct Tracer
             const float nbx = __builtin_fmaf(ox, r.ix, r.cnx), fbx = __builtin_fmaf(ox, r.ix, r.cfx);
             const float nby = __builtin_fmaf(oy, r.iy, r.cny), fby = __builtin_fmaf(oy, r.iy, r.cfy);
             const float nbz = __builtin_fmaf(oz, r.iz, r.cnz), fbz = __builtin_fmaf(oz, r.iz, r.cfz);
-            const bool p0 = qslab_c(r, ch.x, nx, fx, ny, fy, nz, fz, ax, ay, az, nbx, fbx, nby, fby, nbz, fbz, 0, R1, l0);
-            const bool p1 = qslab_c(r, ch.y, nx, fx, ny, fy, nz, fz, ax, ay, az, nbx, fbx, nby, fby, nbz, fbz, 8, R1, l1);
-            const bool p2 = qslab_c(r, ch.z, nx, fx, ny, fy, nz, fz, ax, ay, az, nbx, fbx, nby, fby, nbz, fbz, 16, R1, l2);
-            const bool p3 = qslab_c(r, ch.w, nx, fx, ny, fy, nz, fz, ax, ay, az, nbx, fbx, nby, fby, nbz, fbz, 24, R1, l3);
+            const bool p0 = qslab_c(r, nx, fx, ny, fy, nz, fz, ax, ay, az, nbx, fbx, nby, fby, nbz, fbz, 0, R1, l0);
+            const bool p1 = qslab_c(r, nx, fx, ny, fy, nz, fz, ax, ay, az, nbx, fbx, nby, fby, nbz, fbz, 8, R1, l1);
+            const bool p2 = qslab_c(r, nx, fx, ny, fy, nz, fz, ax, ay, az, nbx, fbx, nby, fby, nbz, fbz, 16, R1, l2);
+            const bool p3 = qslab_c(r, nx, fx, ny, fy, nz, fz, ax, ay, az, nbx, fbx, nby, fby, nbz, fbz, 24, R1, l3);
             // Each slot's position in this octant's visit order; the passing
             // children as a mask over positions.  The nearest is visited
             // next; the others go on the stack farthest first, i.e. a child
@@ -489,7 +497,7 @@ template <bool ANY, bool COUNT>
 MCRT_HD int trace(const DevScene& S, TraceStack& st, const RayPrep& r, float tmax,
                   float& t_out, float& u_out, float& v_out, TraceCount& cnt)
 {
-    Tracer<ANY, COUNT> tr;
+    Tracer<ANY, COUNT, true> tr;
     RayPrep rm = r;
     node_margin(rm, S.node_span);
     tr.start(rm, tmax);

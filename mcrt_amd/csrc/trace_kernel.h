@@ -82,7 +82,7 @@ struct TraceBatch
 // registers into vector lanes, and the spill code in the refill block costs
 // more than the eighth wave gains).  Deeper stacks are held to fewer waves
 // by LDS.
-template <int D, bool ANY, bool COUNT, bool SEG, bool BATCH, bool ORDER>
+template <int D, bool ANY, bool COUNT, bool SEG, bool BATCH, bool ORDER, bool BIG>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     D <= 8 ? (ANY ? kTraceAnyWavesPerSimd : kTraceWavesPerSimd) : 4, 8))) void k_trace(DevScene S, const float4* __restrict__ rays, int64_t n,
                                                  const uint32_t* __restrict__ seg_cnt, int64_t seg1, int64_t seg2,
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     TraceCount cnt;
     uint32_t nrays = 0;
     const uint32_t lane = threadIdx.x;
-    Tracer<ANY, COUNT> tr;
+    Tracer<ANY, COUNT, BIG> tr;
     SceneRoot root;
     root.nodes = S.nodes;
     root.det_eps = S.det_eps;
@@ -253,22 +253,28 @@ inline void launch_k_trace(const DevScene& S, int64_t blocks, hipStream_t st, co
                            unsigned long long* counters, uint32_t* wq, TraceBatch B = TraceBatch())
 {
     const dim3 g((unsigned)blocks), b(kWave);
+    if (S.big)
+    {
+        hipLaunchKernelGGL((k_trace<8, ANY, COUNT, SEG, BATCH, ORDER, true>), g, b, 0, st, S, rays, n, seg_cnt, seg1,
+                           seg2, hits, occ, counters, B, wq);
+        return;
+    }
     switch (S.lds_depth)
     {
     case 8:
-        hipLaunchKernelGGL((k_trace<8, ANY, COUNT, SEG, BATCH, ORDER>), g, b, 0, st, S, rays, n, seg_cnt, seg1, seg2, hits, occ,
+        hipLaunchKernelGGL((k_trace<8, ANY, COUNT, SEG, BATCH, ORDER, false>), g, b, 0, st, S, rays, n, seg_cnt, seg1, seg2, hits, occ,
                            counters, B, wq);
         break;
     case 12:
-        hipLaunchKernelGGL((k_trace<12, ANY, COUNT, SEG, BATCH, ORDER>), g, b, 0, st, S, rays, n, seg_cnt, seg1, seg2, hits, occ,
+        hipLaunchKernelGGL((k_trace<12, ANY, COUNT, SEG, BATCH, ORDER, false>), g, b, 0, st, S, rays, n, seg_cnt, seg1, seg2, hits, occ,
                            counters, B, wq);
         break;
     case 24:
-        hipLaunchKernelGGL((k_trace<24, ANY, COUNT, SEG, BATCH, ORDER>), g, b, 0, st, S, rays, n, seg_cnt, seg1, seg2, hits, occ,
+        hipLaunchKernelGGL((k_trace<24, ANY, COUNT, SEG, BATCH, ORDER, false>), g, b, 0, st, S, rays, n, seg_cnt, seg1, seg2, hits, occ,
                            counters, B, wq);
         break;
     default:
-        hipLaunchKernelGGL((k_trace<16, ANY, COUNT, SEG, BATCH, ORDER>), g, b, 0, st, S, rays, n, seg_cnt, seg1, seg2, hits, occ,
+        hipLaunchKernelGGL((k_trace<16, ANY, COUNT, SEG, BATCH, ORDER, false>), g, b, 0, st, S, rays, n, seg_cnt, seg1, seg2, hits, occ,
                            counters, B, wq);
         break;
     }

@@ -350,13 +350,34 @@ float qnode_span(const std::vector<QNode>& q)
 
 bool device_records(const WideBVH& wb, std::vector<QNode>& nodes_out)
 {
-    const uint64_t nq = wb.qnodes.size();
+    const uint64_t nq = wb.qnodes.size() + 1;  // and the reference of empty slots
     if (nq + wb.refs.size() > (uint64_t)MCRT_LEAF_REF_MASK + 1u) return false;
     nodes_out = wb.qnodes;
     for (QNode& q : nodes_out)
         for (int c = 0; c < 4; c++)
-            if (q.child[c] != MCRT_CHILD_EMPTY && (q.child[c] & MCRT_CHILD_LEAF))
+        {
+            const uint32_t byte = 0xffu << (8 * c);
+            if (q.child[c] == MCRT_CHILD_EMPTY)
+            {
+                q.child[c] = MCRT_CHILD_LEAF | (uint32_t)(nq - 1);
+                for (uint32_t* lo : {&q.q_lo_x, &q.q_lo_y, &q.q_lo_z}) *lo |= byte;
+                for (uint32_t* hi : {&q.q_hi_x, &q.q_hi_y, &q.q_hi_z}) *hi &= ~byte;
+            }
+            else if (q.child[c] & MCRT_CHILD_LEAF)
                 q.child[c] += (uint32_t)nq;  // stays below bit 29: every reference index + nq fits
+        }
+    // an inverted infinite box around a triangle without area
+    WRef none;
+    std::memset(&none, 0, sizeof(none));
+    for (int a = 0; a < 3; a++)
+    {
+        none.lo[a] = std::numeric_limits<float>::infinity();
+        none.hi[a] = -none.lo[a];
+    }
+    none.prim = -1;
+    static_assert(sizeof(QNode) == sizeof(WRef), "nodes and references are records of one array");
+    nodes_out.emplace_back();
+    std::memcpy(static_cast<void*>(&nodes_out.back()), &none, sizeof(none));
     return true;
 }
 
