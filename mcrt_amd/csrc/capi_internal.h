@@ -146,8 +146,8 @@ struct mcrt_scene
     int32_t trace_lds_depth = 8;
     int32_t pt_trace_waves_per_cu = 0;
     int32_t pt_trace_lds_depth = 8;
-    // 2^26 paths per chunk (a whole 1024^2 x 64-spp frame; about 27.9 GB
-    // of path state, 42.3 GB with an environment map): fewer, larger launches
+    // 2^26 paths per chunk (a whole 1024^2 x 64-spp frame; about 25.2 GB
+    // of path state, 33.3 GB with an environment map): fewer, larger launches
     // whose ragged ends weigh less (the frame 109 ms, against 121 ms in 2^24
     // chunks and 140 ms in 2^23)
     int64_t pt_chunk_paths = int64_t(1) << 26;

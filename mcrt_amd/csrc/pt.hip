@@ -60,19 +60,43 @@ namespace mcrt
 namespace
 {
 constexpr int kTPB = 256;
+static_assert(kSegTmin == kEpsRay, "the traversal knows the limit of the path tracer rays");
+
+// Rays of the path tracer: every one has tmin = kEpsRay and no tmax, so a ray
+// is six floats, {o, d.x} and {d.y, d.z}, 24 B where a query's ray has 32.
+// With the throughput in queue order beside its path id (one coalesced load
+// that waits for nothing, where it was a gather by path) and one word instead
+// of a hit per shadow ray: k_direct 4.23 -> 3.66 ms, generate 0.71 -> 0.60,
+// the extend launches 43.8 -> 43.4 of the 1024 x 1024 x 64-spp frame, the
+// batch of 12 scenes 17.25 -> 16.85 ms, 40 B of state less per path (80 B
+// with an environment map).
+struct RaySoA
+{
+    float4* od;
+    float2* d;
+};
+__device__ __forceinline__ V3f ray_dir(const RaySoA& r, int64_t i)
+{
+    const float2 b = r.d[i];
+    return V3f{r.od[i].w, b.x, b.y};
+}
 
 struct PTState
 {
-    float4* T;           // throughput (xyz), w = 1 where the vertex it left was diffuse
+    float4* T;           // environment map: throughput (xyz) per path, w = 1 where the vertex
+                         // it left was diffuse
     float4* L;           // radiance (xyz)
-    float4* rays[2];     // [P continuation | rec_rays(rs) P next-event at the records' slots |
+    RaySoA rays[2];      // [P continuation | rec_rays(rs) P next-event at the records' slots |
                          //  P BSDF-sampled next-event, compacted] x 2 float4 per ray
-    uint32_t* act[2];    // path id per continuation ray
+    uint32_t* act[2];    // environment map: path id per continuation ray
+    float4* tq[2];       // else: per continuation ray its path's throughput and, in w, the
+                         // path id with kDiffuseBit where the vertex it left was diffuse
     float4* rec[2];      // next-event records, rec_words(rs) float4 each
     float4* sh[2];       // no environment map: per light-sample shadow ray the
                          // radiance {x, y, z} it adds to path w where it reaches its
                          // light (w = ~0: the vertex has a record, which adds it)
     uint32_t* want[2];   // and the light triangle it must hit
+    int32_t* sprim;      // and the triangle it hits (or -1)
     float4* shg[2];      // adjoint: and that triangle's emission gradient, its hot slot in w
     uint32_t* bsl[2];    // with an environment map: each record's BSDF-sampled ray slot or ~0
                          // (its 64 B record has no spare word)
@@ -136,10 +160,12 @@ struct PTArgs
     ScenePT one;            // single scene
 };
 
-__device__ __forceinline__ void store_ray(float4* rays, int64_t i, V3f o, V3f d, float tmin, float tmax)
+constexpr uint32_t kDiffuseBit = 1u << 31;  // a path id is below 2^28
+
+__device__ __forceinline__ void store_ray(const RaySoA& rays, int64_t i, V3f o, V3f d)
 {
-    rays[2 * i] = make_float4(o.x, o.y, o.z, tmin);
-    rays[2 * i + 1] = make_float4(d.x, d.y, d.z, tmax);
+    rays.od[i] = make_float4(o.x, o.y, o.z, d.x);
+    rays.d[i] = make_float2(d.y, d.z);
 }
 __device__ __forceinline__ V3f f3(float4 v) { return V3f{v.x, v.y, v.z}; }
 
@@ -374,22 +400,20 @@ __global__ void k_generate(PTState S, PTArgs a)
         // camera ray p is path p, its throughput is one and no earlier
         // vertex was diffuse: the first k_shade takes these as constants,
         // so only the ray and the radiance are stored
-        store_ray(S.rays[0], p, ld3(cam.o), d, kEpsRay, __builtin_inff());
+        store_ray(S.rays[0], p, ld3(cam.o), d);
         S.L[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
 }
 
-// Area-light terms of a next-event record (demo_pt.cpp:591-643 with
-// Scene::lightPdfW scene.cpp:239-267 and lightRadiance :345-366): the
-// BSDF-sampled ray hitting an emitter, MIS-weighted against the light pdf,
-// then the light sample if its shadow ray reaches the sampled light.
-// em1/em2, hot1/hot2 and the coefficients c1/c2 of the two emissions are
-// what the adjoint scatters.
-// rb / rl: the BSDF-sampled ray and the light sample's shadow ray (2 float4
-// each, the direction in the second; read only where the ray hit).
-__device__ __forceinline__ V3f area_terms(const DevScene& D, const int4 h1, const int4 h2, V3f col,
-                                          const float4* rb, const float4* rl, float pdf_b, float factor2, int li,
-                                          V3f local, int& em1,
+// Area-light terms of a diffuse vertex (demo_pt.cpp:591-643 with
+// Scene::lightPdfW scene.cpp:239-267 and lightRadiance :345-366), added to
+// `local` in the reference's order: the BSDF-sampled ray (slot ib of the
+// rays, read only where it hit) hitting an emitter, MIS-weighted against the
+// light pdf, then the light sample (li >= 0: there is one) where its shadow
+// ray reached triangle `lit` (-1: it did not).  em1 / em2, hot1 / hot2 and
+// the coefficients c1 / c2 of the two emissions are what the adjoint scatters.
+__device__ __forceinline__ V3f area_terms(const DevScene& D, const int4 h1, int lit, V3f col, const RaySoA& rays,
+                                          int64_t ib, float pdf_b, float factor2, int li, V3f local, int& em1,
                                           int& em2, int& hot1, int& hot2, V3f& c1, V3f& c2)
 {
     float pdf_l = 0.0f;
@@ -401,7 +425,7 @@ __device__ __forceinline__ V3f area_terms(const DevScene& D, const int4 h1, cons
         if (mt.type == MCRT_LGHT)
         {
             const V3f ns1 = shading_normal(ts, float_of((uint32_t)h1.z), float_of((uint32_t)h1.w));
-            const V3f wb = f3(rb[1]);
+            const V3f wb = ray_dir(rays, ib);
             const float cosl = dot(ns1, -wb);
             if (!(cosl < 1e-6f))
             {
@@ -425,21 +449,12 @@ __device__ __forceinline__ V3f area_terms(const DevScene& D, const int4 h1, cons
     if (li >= 0)
     {
         V3f le2 = v3f(0.0f, 0.0f, 0.0f);
-        if (h2.x >= 0)
+        if (lit >= 0)
         {
-            const TriShade ts = D.shade[h2.x];
-            const DevMaterial mt = D.mats[ts.mat];
-            if (mt.type == MCRT_LGHT)
-            {
-                const V3f ns2 = shading_normal(ts, float_of((uint32_t)h2.z), float_of((uint32_t)h2.w));
-                const V3f wo = f3(rl[1]);
-                if (!(dot(ns2, -wo) < 0) && ts.light == li)
-                {
-                    le2 = ld3(mt.rgb);
-                    em2 = h2.x;
-                    hot2 = ts.hot;
-                }
-            }
+            const TriShade ts = D.shade[lit];
+            le2 = ld3(D.mats[ts.mat].rgb);
+            em2 = lit;
+            hot2 = ts.hot;
         }
         const float ip = 1.0f / kPi;
         f = v3f(ip, ip, ip) * col;  // LambertianBSDF::evaluate (bsdf.cpp:96-116)
@@ -449,21 +464,31 @@ __device__ __forceinline__ V3f area_terms(const DevScene& D, const int4 h1, cons
     return local;
 }
 
+// The triangle that a light sample's shadow ray (slot i, hit h) reached when
+// it is light li's and faces the ray, else -1 (lightRadiance).
+__device__ __forceinline__ int reached(const DevScene& D, const int4 h, const RaySoA& rays, int64_t i, int li)
+{
+    if (h.x < 0) return -1;
+    const TriShade ts = D.shade[h.x];
+    if (D.mats[ts.mat].type != MCRT_LGHT || ts.light != li) return -1;
+    const V3f ns = shading_normal(ts, float_of((uint32_t)h.z), float_of((uint32_t)h.w));
+    return dot(ns, -ray_dir(rays, i)) < 0 ? -1 : h.x;
+}
+
 // Next-event contributions of one diffuse vertex: the environment terms
 // (demo_pt.cpp:564-589), each counted when its shadow ray escapes, then the
-// area-light terms, in the reference's order of accumulation.  ENV: the
-// records hold the environment terms (rs = 4).
-template <bool ADJ, bool BATCH, bool ENV>
+// area-light terms, in the reference's order of accumulation.
+template <bool ADJ, bool BATCH>
 __global__ void k_resolve(PTArgs a, PTState S, int cur)
 {
     __shared__ float acc[ADJ ? 2 * kHotFloats : 1];
     if (ADJ) hot_clear(acc);
     set_counts(S.cnt[cur ^ 1], 0u);
     const int64_t P = a.P;
-    constexpr int rs = ENV ? 4 : 2, rf = rec_rays(rs);
+    constexpr int rs = 4, rf = rec_rays(rs);
     const uint32_t nrec = S.cnt[cur][1] / (uint32_t)rf;
     const float4* R = S.rec[cur];
-    const float4* rays = S.rays[cur];
+    const RaySoA rays = S.rays[cur];
     for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < nrec; base += (int64_t)gridDim.x * blockDim.x)
     {
         const int64_t m = base + threadIdx.x;
@@ -473,31 +498,28 @@ __global__ void k_resolve(PTArgs a, PTState S, int cur)
         if (act)
         {
             const float4* Rm = R + rec_words(rs) * m;
-            const float4 r0 = Rm[0], r1 = Rm[1], r2 = Rm[2], r3 = ENV ? Rm[3] : r2;
+            const float4 r0 = Rm[0], r1 = Rm[1], r2 = Rm[2], r3 = Rm[3];
             const V3f T = f3(r0), col = f3(r1);
-            const uint32_t path = bits_of(ENV ? r2.w : r2.x);
+            const uint32_t path = bits_of(r2.w);
             const DevScene& D = BATCH ? a.tab[S.sid[path]].D : a.one.D;
             const int64_t h0 = P + rf * m;  // the record's first ray slot
             V3f local = v3f(0.0f, 0.0f, 0.0f);
-            if (ENV)
-            {
-                const V3f z = v3f(0.0f, 0.0f, 0.0f);
-                const V3f e1 = S.hits[h0 + 1].x < 0 ? f3(r2) : z;
-                const V3f e2 = S.hits[h0 + 2].x < 0 ? f3(r3) : z;
-                local = local + (e1 + e2);
-            }
+            const V3f z = v3f(0.0f, 0.0f, 0.0f);
+            const V3f e1 = S.hits[h0 + 1].x < 0 ? f3(r2) : z;
+            const V3f e2 = S.hits[h0 + 2].x < 0 ? f3(r3) : z;
+            local = local + (e1 + e2);
             if (D.nlights > 0)
             {
-                const int li = (int)bits_of(ENV ? r3.w : r2.y);
+                const int li = (int)bits_of(r3.w);
                 const int4 miss = make_int4(-1, 0, 0, 0);
                 // the BSDF-sampled ray in the compacted segment after the
                 // records' slots where it was traced, else a miss; the light
                 // sample's shadow ray at the record's first slot
-                const int bs = ENV ? (int)S.bsl[cur][m] : (int)bits_of(r2.z);
+                const int bs = (int)S.bsl[cur][m];
                 const int64_t hb = P + rf * P + bs;
                 V3f c1, c2;
-                local = area_terms(D, bs >= 0 ? S.hits[hb] : miss, li >= 0 ? S.hits[h0] : miss, col, rays + 2 * hb,
-                                   rays + 2 * h0, r0.w, r1.w, li, local, em1, em2, hot1, hot2, c1, c2);
+                local = area_terms(D, bs >= 0 ? S.hits[hb] : miss, li >= 0 ? reached(D, S.hits[h0], rays, h0, li) : -1,
+                                   col, rays, hb, r0.w, r1.w, li, local, em1, em2, hot1, hot2, c1, c2);
                 if (ADJ)
                 {
                     const V3f dl = f3(S.delta[path]);
@@ -577,13 +599,14 @@ __device__ __forceinline__ void env_terms(const DevScene& D, uint64_t key, V3f n
 // reaches none, and its terms are a miss's: it is not traced.  Rays with an
 // infinite inv_dir take the reference's NaN-prone sequential test and are
 // always traced.
-__device__ __forceinline__ void vertex_dirs(const DevScene& D, const float4* rays, int64_t j, int4 h, const TriShade& ts,
+__device__ __forceinline__ void vertex_dirs(const DevScene& D, const RaySoA& rays, int64_t j, int4 h, const TriShade& ts,
                                             bool want_rec, uint64_t key, V3f& d, V3f& phit, V3f& ns, V3f& wb,
                                             bool& trace_wb)
 {
-    const float4 ra = rays[2 * j], rb = rays[2 * j + 1];
+    const float4 ra = rays.od[j];
+    const float2 rb = rays.d[j];
     const V3f o = f3(ra);
-    d = f3(rb);
+    d = V3f{ra.w, rb.x, rb.y};
     const float t = float_of((uint32_t)h.y), u = float_of((uint32_t)h.z), v = float_of((uint32_t)h.w);
     phit = o + d * t;
     ns = shading_normal(ts, u, v);
@@ -640,23 +663,21 @@ __device__ __forceinline__ LightSample sample_area(const DevScene& D, uint64_t k
     return s;
 }
 
-// One vertex of every live path (demo_pt.cpp:523-651).  ENV: a scene of the
+// One vertex of every live path (demo_pt.cpp:523-651) where a scene of the
 // launch has an environment map (escape radiance, rs = 4 next-event rays);
-// without one the environment code is compiled out, which keeps the
-// kernel's registers, and so its occupancy, those of area lights alone.
-// What a vertex emits -- a next-event record, a continuation ray -- depends
-// only on its material, the parameters and the roulette draw, so it is
-// decided first and the workgroup takes its slots (block_slots) before
-// anything is computed or stored.
-template <bool ADJ, bool BATCH, bool ENV>
+// k_shade_direct renders the others.  What a vertex emits -- a next-event
+// record, a continuation ray -- depends only on its material, the parameters
+// and the roulette draw, so it is decided first and the workgroup takes its
+// slots (block_slots) before anything is computed or stored.
+template <bool ADJ, bool BATCH>
 __global__ void k_shade(PTArgs a, PTState S, int cur, int k)
 {
     __shared__ float acc[ADJ ? 2 * kHotFloats : 1];
     if (ADJ) hot_clear(acc);
-    constexpr int rs = ENV ? 4 : 2, rf = rec_rays(rs);
+    constexpr int rs = 4, rf = rec_rays(rs);
     const int nxt = cur ^ 1;
     const uint32_t A = S.cnt[cur][0];
-    const float4* rays = S.rays[cur];
+    const RaySoA rays = S.rays[cur];
     for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < A; base += (int64_t)gridDim.x * blockDim.x)
     {
         const int64_t j = base + threadIdx.x;
@@ -692,7 +713,7 @@ __global__ void k_shade(PTArgs a, PTState S, int cur, int k)
                     const uint64_t sample = (uint64_t)(sp.sample_offset + p % sp.spp);
                     key = rng_key(sp.seed, (uint64_t)pixel, sample, (uint32_t)k);
                 }
-                want_rec = sp.nee && mt.type == MCRT_DIFF && (D.nlights > 0 || (ENV && D.env_w > 0));
+                want_rec = sp.nee && mt.type == MCRT_DIFF && (D.nlights > 0 || D.env_w > 0);
                 // no continuation after the last vertex, or when the roulette ends the path
                 want_cont = !(k >= sp.max_depth) && !(k >= sp.rr_start && rng_u01(key, 7) >= sp.rr_prob);
             }
@@ -709,7 +730,7 @@ __global__ void k_shade(PTArgs a, PTState S, int cur, int k)
         // atomic.  The first vertex has unit throughput and no predecessor.
         V3f T = v3f(1.0f, 1.0f, 1.0f);
         bool no_direct = true;
-        if (act && k != 0 && (h.x >= 0 || (ENV && D.env_w > 0)))
+        if (act && k != 0 && (h.x >= 0 || D.env_w > 0))
         {
             const float4 t4 = S.T[p];
             T = f3(t4);
@@ -723,9 +744,9 @@ __global__ void k_shade(PTArgs a, PTState S, int cur, int k)
             if (h.x < 0)
             {
                 // escape: the passive environment term (demo_pt.cpp:528-540)
-                if (ENV && D.env_w > 0 && no_direct)
+                if (D.env_w > 0 && no_direct)
                 {
-                    const V3f Lv = f3(S.L[p]) + T * env_rad(D, env_pixel(D, f3(rays[2 * j + 1])));
+                    const V3f Lv = f3(S.L[p]) + T * env_rad(D, env_pixel(D, ray_dir(rays, j)));
                     S.L[p] = f4(Lv);
                 }
                 break;
@@ -762,7 +783,7 @@ __global__ void k_shade(PTArgs a, PTState S, int cur, int k)
                 const int64_t m = rslot / (uint32_t)rf;
                 const int64_t r0i = a.P + (int64_t)rslot;
                 float4* R = S.rec[nxt] + rec_words(rs) * m;
-                float4* nr = S.rays[nxt];
+                const RaySoA nr = S.rays[nxt];
                 const V3f zero = v3f(0.0f, 0.0f, 0.0f);
                 V3f wo = zero;
                 float pdf_b = 1.0f, factor2 = 0.0f;
@@ -778,23 +799,17 @@ __global__ void k_shade(PTArgs a, PTState S, int cur, int k)
                 R[0] = make_float4(T.x, T.y, T.z, pdf_b);
                 R[1] = make_float4(col.x, col.y, col.z, factor2);
                 const uint32_t bs = trace_wb ? bslot : ~0u;
-                if (ENV)
-                    S.bsl[nxt][m] = bs;
-                else
-                    R[2] = make_float4(float_of(p), float_of((uint32_t)li_rec), float_of(bs), 0.0f);
+                S.bsl[nxt][m] = bs;
                 // a zero direction fails every slab test (ray.cpp:77-79): the
                 // rays a vertex does not need cost one root visit
-                store_ray(nr, r0i, phit, li_rec >= 0 ? wo : zero, kEpsRay, __builtin_inff());
-                if (trace_wb) store_ray(nr, a.P + rf * a.P + bslot, phit, wb, kEpsRay, __builtin_inff());
-                if (ENV)
-                {
-                    V3f e1 = zero, e2 = zero, d1 = zero, d2 = zero;
-                    if (D.env_w > 0) env_terms(D, key, ns, col, e1, e2, d1, d2);
-                    R[2] = make_float4(e1.x, e1.y, e1.z, float_of(p));
-                    R[3] = make_float4(e2.x, e2.y, e2.z, float_of((uint32_t)li_rec));
-                    store_ray(nr, r0i + 1, phit, d1, kEpsRay, __builtin_inff());
-                    store_ray(nr, r0i + 2, phit, d2, kEpsRay, __builtin_inff());
-                }
+                store_ray(nr, r0i, phit, li_rec >= 0 ? wo : zero);
+                if (trace_wb) store_ray(nr, a.P + rf * a.P + bslot, phit, wb);
+                V3f e1 = zero, e2 = zero, d1 = zero, d2 = zero;
+                if (D.env_w > 0) env_terms(D, key, ns, col, e1, e2, d1, d2);
+                R[2] = make_float4(e1.x, e1.y, e1.z, float_of(p));
+                R[3] = make_float4(e2.x, e2.y, e2.z, float_of((uint32_t)li_rec));
+                store_ray(nr, r0i + 1, phit, d1);
+                store_ray(nr, r0i + 2, phit, d2);
                 if (BATCH)
                 {
                     for (int i = 0; i < rf; i++) S.rsid[nxt][r0i + i] = sid;
@@ -819,7 +834,7 @@ __global__ void k_shade(PTArgs a, PTState S, int cur, int k)
             T = T * weight;
             if (k >= sp.rr_start) T = T * (1.0f / sp.rr_prob);
             S.T[p] = make_float4(T.x, T.y, T.z, mt.type == MCRT_DIFF ? 1.0f : 0.0f);
-            store_ray(S.rays[nxt], cslot, phit, nd, kEpsRay, __builtin_inff());
+            store_ray(S.rays[nxt], cslot, phit, nd);
             S.act[nxt][cslot] = p;
             if (BATCH) S.rsid[nxt][cslot] = sid;
         } while (false);
@@ -855,7 +870,7 @@ __global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
     if (ADJ) hot_clear(acc);
     const int nxt = cur ^ 1;
     const uint32_t A = S.cnt[cur][0];
-    const float4* rays = S.rays[cur];
+    const RaySoA rays = S.rays[cur];
     for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < A; base += (int64_t)gridDim.x * blockDim.x)
     {
         const int64_t j = base + threadIdx.x;
@@ -863,9 +878,11 @@ __global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
         uint32_t p = 0;
         int4 h = make_int4(-1, 0, 0, 0);
         uint16_t sid = 0;
+        float4 tq = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
         if (act)
         {
-            p = k == 0 ? (uint32_t)j : S.act[cur][j];
+            if (k != 0) tq = S.tq[cur][j];
+            p = k == 0 ? (uint32_t)j : bits_of(tq.w) & ~kDiffuseBit;
             h = S.hits[j];
             if (BATCH) sid = S.sid[p];
         }
@@ -894,14 +911,8 @@ __global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
         V3f d = zero, phit = zero, ns = zero, wb = zero;
         bool trace_wb = false;
         if (hit) vertex_dirs(D, rays, j, h, ts, want_rec, key, d, phit, ns, wb, trace_wb);
-        V3f T = v3f(1.0f, 1.0f, 1.0f);
-        bool no_direct = true;
-        if (hit && k != 0)
-        {
-            const float4 t4 = S.T[p];
-            T = f3(t4);
-            no_direct = !sp.nee || t4.w == 0.0f;
-        }
+        V3f T = f3(tq);
+        const bool no_direct = k == 0 || !sp.nee || (bits_of(tq.w) & kDiffuseBit) == 0;
         const V3f col = ld3(mt.rgb);
         V3f wo = zero, x = zero, c2 = zero;
         float factor2 = 0.0f;
@@ -979,11 +990,11 @@ __global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
             g_alb = v3f(col.x > 0.0f ? dl.x * rest.x / col.x : 0.0f, col.y > 0.0f ? dl.y * rest.y / col.y : 0.0f,
                         col.z > 0.0f ? dl.z * rest.z / col.z : 0.0f);
         }
-        float4* nr = S.rays[nxt];
+        const RaySoA nr = S.rays[nxt];
         if (want_sh)
         {
             const int64_t r1 = a.P + (int64_t)sslot;
-            store_ray(nr, r1, phit, wo, kEpsRay, __builtin_inff());
+            store_ray(nr, r1, phit, wo);
             S.sh[nxt][sslot] = make_float4(x.x, x.y, x.z, float_of(trace_wb ? ~0u : p));
             S.want[nxt][sslot] = (uint32_t)tri;
             if (ADJ)
@@ -1000,7 +1011,7 @@ __global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
             R[0] = make_float4(T.x, T.y, T.z, fmax_ref(dot(wb, ns), kEpsCos) / kPi);
             R[1] = make_float4(col.x, col.y, col.z, factor2);
             R[2] = make_float4(float_of(p), float_of((uint32_t)li), float_of(want_sh ? sslot : ~0u), 0.0f);
-            store_ray(nr, r2, phit, wb, kEpsRay, __builtin_inff());
+            store_ray(nr, r2, phit, wb);
             if (BATCH) S.rsid[nxt][r2] = sid;
         }
         if (want_cont)
@@ -1021,9 +1032,8 @@ __global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
             }
             T = T * weight;
             if (k >= sp.rr_start) T = T * (1.0f / sp.rr_prob);
-            S.T[p] = make_float4(T.x, T.y, T.z, mt.type == MCRT_DIFF ? 1.0f : 0.0f);
-            store_ray(nr, cslot, phit, nd, kEpsRay, __builtin_inff());
-            S.act[nxt][cslot] = p;
+            S.tq[nxt][cslot] = make_float4(T.x, T.y, T.z, float_of(p | (mt.type == MCRT_DIFF ? kDiffuseBit : 0u)));
+            store_ray(nr, cslot, phit, nd);
             if (BATCH) S.rsid[nxt][cslot] = sid;
         }
         if (ADJ)
@@ -1057,7 +1067,7 @@ __global__ void k_direct(PTArgs a, PTState S, int cur)
             const float4 xp = S.sh[cur][s];
             const uint32_t path = bits_of(xp.w);
             const int tri = (int)S.want[cur][s];
-            if (path != ~0u && S.hits[a.P + s].x == tri)
+            if (path != ~0u && S.sprim[s] == tri)
             {
                 const V3f x = f3(xp);
                 // a zero term leaves the path's radiance as it is (k_resolve)
@@ -1073,7 +1083,7 @@ __global__ void k_direct(PTArgs a, PTState S, int cur)
         }
         if (ADJ) grad_add(acc + kHotFloats, S.g_em, em, hot, g, em >= 0);
     }
-    const float4* rays = S.rays[cur];
+    const RaySoA rays = S.rays[cur];
     for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < nrec; base += step)
     {
         const int64_t m = base + threadIdx.x;
@@ -1086,11 +1096,11 @@ __global__ void k_direct(PTArgs a, PTState S, int cur)
             const uint32_t path = bits_of(r2.x);
             const int li = (int)bits_of(r2.y), ss = (int)bits_of(r2.z);
             const DevScene& D = BATCH ? a.tab[S.sid[path]].D : a.one.D;
-            const int64_t hb = 2 * a.P + m, hs = a.P + ss;
+            const int64_t hb = 2 * a.P + m;
+            const int lit = ss >= 0 && S.sprim[ss] == (int)S.want[cur][ss] ? S.sprim[ss] : -1;
             V3f c1, c2;
-            const V3f local = area_terms(D, S.hits[hb], ss >= 0 ? S.hits[hs] : make_int4(-1, 0, 0, 0), f3(r1),
-                                         rays + 2 * hb, rays + 2 * hs, r0.w, r1.w, li, v3f(0.0f, 0.0f, 0.0f), em1,
-                                         em2, hot1, hot2, c1, c2);
+            const V3f local = area_terms(D, S.hits[hb], lit, f3(r1), rays, hb, r0.w, r1.w, li,
+                                         v3f(0.0f, 0.0f, 0.0f), em1, em2, hot1, hot2, c1, c2);
             const V3f T = f3(r0), x = T * local;
             if (!(x.x == 0.0f && x.y == 0.0f && x.z == 0.0f)) S.L[path] = f4(f3(S.L[path]) + x);
             if (ADJ)
@@ -1227,15 +1237,16 @@ void bounce_loop(const DevScene& Dt, PTState& S, const PTArgs& a, int max_depth,
         TraceBatch tb;
         tb.roots = a.roots;
         tb.rsid = S.rsid[cur];
-        launch_k_trace<false, false, true, BATCH>(Dt, trace_blocks(Dt, (1 + a.rs) * a.P), st, S.rays[cur], (int64_t)0,
-                                                  S.cnt[cur], a.P, a.P + rec_rays(a.rs) * a.P, S.hits, (uint8_t*)nullptr,
-                                                  (unsigned long long*)nullptr, S.cnt[cur] + kCntWq, tb);
+        const auto trace = a.rs == 4 ? launch_k_trace<false, false, kSegHits, BATCH>
+                                     : launch_k_trace<false, false, kSegDirect, BATCH>;
+        trace(Dt, trace_blocks(Dt, (1 + a.rs) * a.P), st, S.rays[cur].od, (int64_t)0, S.cnt[cur], a.P,
+              a.P + rec_rays(a.rs) * a.P, S.hits, nullptr, nullptr, S.cnt[cur] + kCntWq, tb);
         if (k == 0)
         {
             // no records yet
         }
         else if (a.rs == 4)
-            hipLaunchKernelGGL((k_resolve<ADJ, BATCH, true>), (grid_of<k_resolve<ADJ, BATCH, true>>(a.P, cus)),
+            hipLaunchKernelGGL((k_resolve<ADJ, BATCH>), (grid_of<k_resolve<ADJ, BATCH>>(a.P, cus)),
                                dim3(kTPB), 0, st, a, S, cur);
         else
             hipLaunchKernelGGL((k_direct<ADJ, BATCH>), (grid_of<k_direct<ADJ, BATCH>>(a.P, cus)), dim3(kTPB), 0, st, a,
@@ -1243,7 +1254,7 @@ void bounce_loop(const DevScene& Dt, PTState& S, const PTArgs& a, int max_depth,
         if (k <= max_depth)
         {
             if (a.rs == 4)
-                hipLaunchKernelGGL((k_shade<ADJ, BATCH, true>), (grid_of<k_shade<ADJ, BATCH, true>>(a.P, cus)),
+                hipLaunchKernelGGL((k_shade<ADJ, BATCH>), (grid_of<k_shade<ADJ, BATCH>>(a.P, cus)),
                                    dim3(kTPB), 0, st, a, S, cur, k);
             else
                 hipLaunchKernelGGL((k_shade_direct<ADJ, BATCH>), (grid_of<k_shade_direct<ADJ, BATCH>>(a.P, cus)),
@@ -1253,8 +1264,8 @@ void bounce_loop(const DevScene& Dt, PTState& S, const PTArgs& a, int max_depth,
     }
 }
 
-// The path state of chunks of at most P paths.
-PTState state_of(StreamRes* r, int64_t P, bool adjoint)
+// The path state of a chunk of P paths.
+PTState state_of(StreamRes* r, int64_t P, bool adjoint, int rs)
 {
     PTWork& w = r->ptw;
     PTState S;
@@ -1262,8 +1273,10 @@ PTState state_of(StreamRes* r, int64_t P, bool adjoint)
     S.L = w.L.as<float4>();
     for (int i = 0; i < 2; i++)
     {
-        S.rays[i] = w.rays[i].as<float4>();
+        S.rays[i].od = w.rays[i].as<float4>();
+        S.rays[i].d = reinterpret_cast<float2*>(S.rays[i].od + seg_cap(rs == 4 ? kSegHits : kSegDirect, P));
         S.act[i] = w.act[i].as<uint32_t>();
+        S.tq[i] = w.act[i].as<float4>();
         S.rec[i] = w.rec[i].as<float4>();
         S.bsl[i] = w.bsl[i].as<uint32_t>();
         // the shadow rays' terms follow the P records (pt_workspace)
@@ -1274,6 +1287,8 @@ PTState state_of(StreamRes* r, int64_t P, bool adjoint)
         S.rsid[i] = w.rsid[i].as<uint16_t>();
     }
     S.hits = w.hits.as<int4>();
+    // the shadow rays' part of the hits holds their triangles alone
+    S.sprim = reinterpret_cast<int32_t*>(S.hits + P);
     S.Ltot = adjoint ? w.Ltot.as<float4>() : nullptr;
     S.delta = adjoint ? w.delta.as<float4>() : nullptr;
     S.g_alb = S.g_em = nullptr;
@@ -1308,12 +1323,12 @@ int pt_workspace(StreamRes* r, int64_t P, bool adjoint, bool batch, int rs)
     PTWork& w = r->ptw;
     int rc;
     const size_t n = (size_t)P, nr = (size_t)(1 + rs) * n;
-    if ((rc = w.T.ensure(n * 16))) return rc;
+    if (rs == 4 && (rc = w.T.ensure(n * 16))) return rc;
     if ((rc = w.L.ensure(n * 16))) return rc;
     for (int i = 0; i < 2; i++)
     {
-        if ((rc = w.rays[i].ensure(nr * 32))) return rc;
-        if ((rc = w.act[i].ensure(n * 4))) return rc;
+        if ((rc = w.rays[i].ensure(nr * 24))) return rc;
+        if ((rc = w.act[i].ensure(n * (rs == 4 ? 4 : 16)))) return rc;
         // without an environment map also the shadow rays' terms and triangles
         // (and, for the adjoint, gradients)
         if ((rc = w.rec[i].ensure(n * (16 * rec_words(rs) + (rs == 4 ? 0 : adjoint ? 36 : 20))))) return rc;
@@ -1351,9 +1366,6 @@ int render_scene(mcrt_scene* s, StreamRes* r, const mcrt_render_params* prm, flo
     if (pix_per_chunk > npix) pix_per_chunk = npix;
     const int rs = D.env_w > 0 ? 4 : 2;
     if ((rc = pt_workspace(r, pix_per_chunk * spp, adj != nullptr, false, rs))) return rc;
-    PTState S = state_of(r, pix_per_chunk * spp, adj != nullptr);
-    S.g_alb = adj ? adj->d_albedo : nullptr;
-    S.g_em = adj ? adj->d_emission : nullptr;
     const int cus = s->ctx->num_cus;
     if (adj)
     {
@@ -1373,6 +1385,9 @@ int render_scene(mcrt_scene* s, StreamRes* r, const mcrt_render_params* prm, flo
         const int64_t np = std::min(pix_per_chunk, npix - pix0);
         a.P = np * spp;
         a.pix0 = pix0;
+        PTState S = state_of(r, a.P, adj != nullptr, rs);
+        S.g_alb = adj ? adj->d_albedo : nullptr;
+        S.g_em = adj ? adj->d_emission : nullptr;
         bounce_loop<false, false>(D, S, a, prm->max_depth, cus, st);
         if (adj)
         {
@@ -1479,9 +1494,6 @@ int batch_init(mcrt_batch* b)
 // Every kernel of the batch on `st` (launches only: capturable).
 int batch_enqueue(mcrt_batch* b, hipStream_t st)
 {
-    int64_t pcap = 0;
-    for (const BatchChunk& c : b->chunks) pcap = std::max(pcap, c.P);
-    PTState S = state_of(&b->res, pcap, false);
     const int cus = b->ctx->num_cus;
     PTArgs a;
     a.pix0 = 0;
@@ -1492,6 +1504,7 @@ int batch_enqueue(mcrt_batch* b, hipStream_t st)
     for (const BatchChunk& c : b->chunks)
     {
         a.P = c.P;
+        PTState S = state_of(&b->res, c.P, false, b->rs);
         a.nseg = (int32_t)c.nseg;
         a.seg = b->d_seg.as<Segment>() + c.seg0;
         bounce_loop<false, true>(b->trace_view, S, a, b->max_depth, cus, st);

@@ -38,8 +38,8 @@
 // 256 were 2-5% slower at 700k to 1M rays.
 //
 // Two ray sources:
-//   * SEG = false: rays[0, n) with n known to the host;
-//   * SEG = true : three segments whose sizes live in device memory (the
+//   * SEG = kQuery: rays[0, n) with n known to the host;
+//   * otherwise three segments whose sizes live in device memory (the
 //     path tracer's compacted continuation rays [0, cnt[0]), its next-event
 //     rays at their records' slots [seg1, seg1 + cnt[1]) and its compacted
 //     BSDF-sampled next-event rays [seg2, seg2 + cnt[kSeg2Word])), so the
@@ -75,6 +75,19 @@ struct TraceBatch
     const uint32_t* order = nullptr;
     const uint32_t* skip = nullptr;
 };
+// Ray sources of a launch: a query's rays, or the path tracer's segments,
+// whose rays are {o, d.x} and, from seg_cap(seg1) rays on, {d.y, d.z}, all
+// with tmin = kSegTmin (NUM_EPS_RAY) and no tmax.  kSegDirect: the second
+// segment holds shadow rays of which only the triangle they hit matters; it
+// is stored alone, as one word per ray from hits[seg1] on.
+enum RaySource
+{
+    kQuery = 0,
+    kSegHits = 1,   // with an environment map: five rays per path
+    kSegDirect = 2  // without: three
+};
+__host__ __device__ constexpr int64_t seg_cap(int seg, int64_t paths) { return (seg == kSegDirect ? 3 : 5) * paths; }
+constexpr float kSegTmin = 1e-4f;
 
 // With an 8-entry stack the closest-hit kernel is compiled for eight waves
 // per SIMD (32 per CU, with LDS for all of them: 64 VGPRs), the any-hit
@@ -82,7 +95,7 @@ struct TraceBatch
 // registers into vector lanes, and the spill code in the refill block costs
 // more than the eighth wave gains).  Deeper stacks are held to fewer waves
 // by LDS.
-template <int D, bool ANY, bool COUNT, bool SEG, bool BATCH, bool ORDER, bool BIG>
+template <int D, bool ANY, bool COUNT, int SEG, bool BATCH, bool ORDER, bool BIG>
 __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     D <= 8 ? (ANY ? kTraceAnyWavesPerSimd : kTraceWavesPerSimd) : 4, 8))) void k_trace(DevScene S, const float4* __restrict__ rays, int64_t n,
                                                  const uint32_t* __restrict__ seg_cnt, int64_t seg1, int64_t seg2,
@@ -193,10 +206,21 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
                 else
                     i = (ORDER && order != nullptr) ? order[k] : k;
                 if (BATCH) root = B.roots[B.rsid[i]];
-                const float4 a = rays[2 * (size_t)i], b = rays[2 * (size_t)i + 1];
-                RayPrep rp = prep_ray(a.x, a.y, a.z, b.x, b.y, b.z, a.w);
-                node_margin(rp, root.node_span);
-                tr.start(rp, b.w);
+                if (SEG)
+                {
+                    const float4 a = rays[i];
+                    const float2 b = reinterpret_cast<const float2*>(rays + seg_cap(SEG, seg1))[i];
+                    RayPrep rp = prep_ray(a.x, a.y, a.z, a.w, b.x, b.y, kSegTmin);
+                    node_margin(rp, root.node_span);
+                    tr.start(rp, __builtin_inff());
+                }
+                else
+                {
+                    const float4 a = rays[2 * (size_t)i], b = rays[2 * (size_t)i + 1];
+                    RayPrep rp = prep_ray(a.x, a.y, a.z, b.x, b.y, b.z, a.w);
+                    node_margin(rp, root.node_span);
+                    tr.start(rp, b.w);
+                }
                 live = true;
             }
             const uint32_t nidle = (uint32_t)__popcll(idle);
@@ -217,6 +241,8 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
             const int prim = tr.result(t, u, v);
             if (ANY)
                 occ[i] = prim >= 0 ? 1 : 0;
+            else if (SEG == kSegDirect && i >= (uint32_t)seg1 && i < (uint32_t)seg2)
+                reinterpret_cast<int32_t*>(hits + seg1)[i - (uint32_t)seg1] = prim;
             else
                 hits[i] = make_int4(prim, (int)bits_of(t), (int)bits_of(u), (int)bits_of(v));
             nrays++;
@@ -247,7 +273,7 @@ inline int64_t trace_blocks(const DevScene& s, int64_t n)
 
 // Launches k_trace with the scene's LDS stack depth on `blocks` workgroups;
 // wq holds kWqWords words, the slice counters zero.
-template <bool ANY, bool COUNT, bool SEG, bool BATCH = false, bool ORDER = false>
+template <bool ANY, bool COUNT, int SEG, bool BATCH = false, bool ORDER = false>
 inline void launch_k_trace(const DevScene& S, int64_t blocks, hipStream_t st, const float4* rays, int64_t n,
                            const uint32_t* seg_cnt, int64_t seg1, int64_t seg2, int4* hits, uint8_t* occ,
                            unsigned long long* counters, uint32_t* wq, TraceBatch B = TraceBatch())
