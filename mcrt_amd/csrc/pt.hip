@@ -60,6 +60,20 @@ namespace mcrt
 namespace
 {
 constexpr int kTPB = 256;
+// Largest workgroup of the shading kernels.  Each iteration of a workgroup
+// takes its slots with atomics on one address, which serialise at about 11.7
+// ns, so the launch over 2^26 camera paths cannot end before 67.1 M / threads
+// x 11.7 ns: with 256 threads 3.07 ms of the 3.19 ms it took, with 128 threads
+// twice that.  With 512 it takes 2.4 ms, bound by its loads and stores; with
+// 1,024 the workgroups' barriers cost what the atomics save.  The forward
+// kernel is held to 80 registers (6 waves per SIMD, a few spilled): frame
+// 62.2 -> 58.4 ms, against 59.8 ms at 5 waves; the adjoint's is left at 5
+// (held to 6 its step takes 18.4 instead of 17.2 ms).  Launches that do not
+// fill the chip with workgroups of 512 (kShadeLarge paths) and the batched
+// kernels, whose per-path lookups keep them off the atomics, run 256 (97x61
+// frame 520 against 528 us, batch of 12 scenes 16.85 against 17.06 ms).
+constexpr int kShadeTPB = 512;
+constexpr int64_t kShadeLarge = int64_t(1) << 18;
 static_assert(kSegTmin == kEpsRay, "the traversal knows the limit of the path tracer rays");
 
 // Rays of the path tracer: every one has tmin = kEpsRay and no tmax, so a ray
@@ -184,8 +198,7 @@ __device__ __forceinline__ V3f f3(float4 v) { return V3f{v.x, v.y, v.z}; }
 __device__ __forceinline__ void block_slots(uint32_t* c, bool a, bool b, bool e, uint32_t per, uint32_t& sa,
                                             uint32_t& sb, uint32_t& se)
 {
-    constexpr uint32_t W = kTPB / 64;
-    __shared__ uint32_t s_n[3][W];
+    __shared__ uint32_t s_n[3][kShadeTPB / 64];
     __shared__ unsigned long long s_base;
     __shared__ uint32_t s_base_e;
     const uint64_t ma = __ballot(a), mb = __ballot(b), me = __ballot(e);
@@ -198,7 +211,7 @@ __device__ __forceinline__ void block_slots(uint32_t* c, bool a, bool b, bool e,
     }
     __syncthreads();
     uint32_t pa = 0, pb = 0, pe = 0, ta = 0, tb = 0, te = 0;
-    for (uint32_t q = 0; q < W; q++)
+    for (uint32_t q = 0; q < blockDim.x / 64; q++)
     {
         const uint32_t na = s_n[0][q], nb = s_n[1][q], ne = s_n[2][q];
         pa += q < w ? na : 0u;
@@ -670,7 +683,7 @@ __device__ __forceinline__ LightSample sample_area(const DevScene& D, uint64_t k
 // and the roulette draw, so it is decided first and the workgroup takes its
 // slots (block_slots) before anything is computed or stored.
 template <bool ADJ, bool BATCH>
-__global__ void k_shade(PTArgs a, PTState S, int cur, int k)
+__global__ __launch_bounds__(kShadeTPB) void k_shade(PTArgs a, PTState S, int cur, int k)
 {
     __shared__ float acc[ADJ ? 2 * kHotFloats : 1];
     if (ADJ) hot_clear(acc);
@@ -864,7 +877,8 @@ __global__ void k_shade(PTArgs a, PTState S, int cur, int k)
 // instead of 86 registers (6 waves per SIMD).  Bound by the latency of its
 // dependent loads (path, hit, triangle, material) and by its stores.
 template <bool ADJ, bool BATCH>
-__global__ void k_shade_direct(PTArgs a, PTState S, int cur, int k)
+__global__ __launch_bounds__(kShadeTPB) __attribute__((amdgpu_waves_per_eu(ADJ || BATCH ? 5 : 6, 8))) void k_shade_direct(
+    PTArgs a, PTState S, int cur, int k)
 {
     __shared__ float acc[ADJ ? 2 * kHotFloats : 1];
     if (ADJ) hot_clear(acc);
@@ -1194,14 +1208,14 @@ __global__ void k_accumulate(PTState S, PTArgs a, float* film, int64_t npix)
     }
 }
 
-// Workgroups of kTPB threads of kernel K resident at once on a CU (queried
+// Workgroups of TPB threads of kernel K resident at once on a CU (queried
 // once per kernel).
-template <auto K>
+template <auto K, int TPB>
 int resident_per_cu()
 {
     static const int n = [] {
         int b = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, reinterpret_cast<const void*>(K), kTPB, 0) != hipSuccess)
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, reinterpret_cast<const void*>(K), TPB, 0) != hipSuccess)
         {
             (void)hipGetLastError();
             b = 0;
@@ -1215,11 +1229,11 @@ int resident_per_cu()
 // are resident at once, so all of them start together and none is left
 // for a second round (a grid a little larger than what fits doubles the
 // time of its last workgroups).
-template <auto K>
+template <auto K, int TPB = kTPB>
 dim3 grid_of(int64_t n, int num_cus)
 {
-    int64_t b = (n + kTPB - 1) / kTPB;
-    const int64_t cap = (int64_t)num_cus * resident_per_cu<K>();
+    int64_t b = (n + TPB - 1) / TPB;
+    const int64_t cap = (int64_t)num_cus * resident_per_cu<K, TPB>();
     if (b > cap) b = cap;
     if (b < 1) b = 1;
     return dim3((unsigned)b);
@@ -1253,12 +1267,18 @@ void bounce_loop(const DevScene& Dt, PTState& S, const PTArgs& a, int max_depth,
                                S, cur);
         if (k <= max_depth)
         {
+            const bool large = !BATCH && a.P >= kShadeLarge;
+            const dim3 threads(large ? kShadeTPB : kTPB);
             if (a.rs == 4)
-                hipLaunchKernelGGL((k_shade<ADJ, BATCH>), (grid_of<k_shade<ADJ, BATCH>>(a.P, cus)),
-                                   dim3(kTPB), 0, st, a, S, cur, k);
+                hipLaunchKernelGGL((k_shade<ADJ, BATCH>),
+                                   (large ? grid_of<k_shade<ADJ, BATCH>, kShadeTPB>(a.P, cus)
+                                          : grid_of<k_shade<ADJ, BATCH>>(a.P, cus)),
+                                   threads, 0, st, a, S, cur, k);
             else
-                hipLaunchKernelGGL((k_shade_direct<ADJ, BATCH>), (grid_of<k_shade_direct<ADJ, BATCH>>(a.P, cus)),
-                                   dim3(kTPB), 0, st, a, S, cur, k);
+                hipLaunchKernelGGL((k_shade_direct<ADJ, BATCH>),
+                                   (large ? grid_of<k_shade_direct<ADJ, BATCH>, kShadeTPB>(a.P, cus)
+                                          : grid_of<k_shade_direct<ADJ, BATCH>>(a.P, cus)),
+                                   threads, 0, st, a, S, cur, k);
         }
         cur ^= 1;
     }
