@@ -181,6 +181,13 @@ __device__ __forceinline__ void store_ray(const RaySoA& rays, int64_t i, V3f o, 
     rays.od[i] = make_float4(o.x, o.y, o.z, d.x);
     rays.d[i] = make_float2(d.y, d.z);
 }
+__device__ __forceinline__ void load_ray(const RaySoA& rays, int64_t i, V3f& o, V3f& d)
+{
+    const float4 a = rays.od[i];
+    const float2 b = rays.d[i];
+    o = V3f{a.x, a.y, a.z};
+    d = V3f{a.w, b.x, b.y};
+}
 __device__ __forceinline__ V3f f3(float4 v) { return V3f{v.x, v.y, v.z}; }
 
 // Slots of this thread in the workgroup's three compactions of one
@@ -366,6 +373,29 @@ __device__ __forceinline__ int find_seg(const Segment* seg, int nseg, int64_t x)
 }
 
 // Camera::makeRay (camera.cpp:37-43) + tent filter (demo_pt.cpp:687-699).
+__device__ __forceinline__ void camera_ray(const ScenePT& sp, int64_t pixel, uint64_t sample, V3f& o, V3f& d)
+{
+    const DevCamera& cam = sp.cam;
+    const int x = (int)(pixel % cam.w), y = (int)(pixel / cam.w);
+    float dx = 0.0f, dy = 0.0f;
+    if (sp.spp > 1)
+    {
+        const uint64_t key = rng_key(sp.seed, (uint64_t)pixel, sample, 255u);
+        float r1 = 2.0f * rng_u01(key, 0);
+        float r2 = 2.0f * rng_u01(key, 1);
+        dx = r1 < 1 ? sqrtf(r1) - 1.0f : 1.0f - sqrtf(2.0f - r1);
+        dy = r2 < 1 ? sqrtf(r2) - 1.0f : 1.0f - sqrtf(2.0f - r2);
+    }
+    float mx = (((float)x + 0.5f) + dx) / (float)cam.w;
+    float my = (((float)y + 0.5f) + dy) / (float)cam.h;
+    V3f su = (ld3(cam.fx) * (mx - 0.5f)) * cam.ww;
+    V3f sv = (ld3(cam.fy) * (my - 0.5f)) * 1.0f;
+    V3f sw = ld3(cam.fwd) * cam.dist;
+    o = ld3(cam.o);
+    d = nrm((su + sv) + sw);
+}
+
+// The camera rays of a chunk.
 template <bool BATCH>
 __global__ void k_generate(PTState S, PTArgs a)
 {
@@ -393,40 +423,25 @@ __global__ void k_generate(PTState S, PTArgs a)
             pixel = a.pix0 + p / a.one.spp;
             sample = (uint64_t)(a.one.sample_offset + p % a.one.spp);
         }
-        const DevCamera& cam = sp->cam;
-        const int x = (int)(pixel % cam.w), y = (int)(pixel / cam.w);
-        float dx = 0.0f, dy = 0.0f;
-        if (sp->spp > 1)
-        {
-            const uint64_t key = rng_key(sp->seed, (uint64_t)pixel, sample, 255u);
-            float r1 = 2.0f * rng_u01(key, 0);
-            float r2 = 2.0f * rng_u01(key, 1);
-            dx = r1 < 1 ? sqrtf(r1) - 1.0f : 1.0f - sqrtf(2.0f - r1);
-            dy = r2 < 1 ? sqrtf(r2) - 1.0f : 1.0f - sqrtf(2.0f - r2);
-        }
-        float mx = (((float)x + 0.5f) + dx) / (float)cam.w;
-        float my = (((float)y + 0.5f) + dy) / (float)cam.h;
-        V3f su = (ld3(cam.fx) * (mx - 0.5f)) * cam.ww;
-        V3f sv = (ld3(cam.fy) * (my - 0.5f)) * 1.0f;
-        V3f sw = ld3(cam.fwd) * cam.dist;
-        V3f d = nrm((su + sv) + sw);
+        V3f o, d;
+        camera_ray(*sp, pixel, sample, o, d);
         // camera ray p is path p, its throughput is one and no earlier
         // vertex was diffuse: the first k_shade takes these as constants,
         // so only the ray and the radiance are stored
-        store_ray(S.rays[0], p, ld3(cam.o), d);
+        store_ray(S.rays[0], p, o, d);
         S.L[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     }
 }
 
 // Area-light terms of a diffuse vertex (demo_pt.cpp:591-643 with
 // Scene::lightPdfW scene.cpp:239-267 and lightRadiance :345-366), added to
-// `local` in the reference's order: the BSDF-sampled ray (slot ib of the
-// rays, read only where it hit) hitting an emitter, MIS-weighted against the
+// `local` in the reference's order: the BSDF-sampled ray (its direction
+// wb_of() is formed only where it hit) hitting an emitter, MIS-weighted against the
 // light pdf, then the light sample (li >= 0: there is one) where its shadow
 // ray reached triangle `lit` (-1: it did not).  em1 / em2, hot1 / hot2 and
 // the coefficients c1 / c2 of the two emissions are what the adjoint scatters.
-__device__ __forceinline__ V3f area_terms(const DevScene& D, const int4 h1, int lit, V3f col, const RaySoA& rays,
-                                          int64_t ib, float pdf_b, float factor2, int li, V3f local, int& em1,
+template <class Dir>
+__device__ __forceinline__ V3f area_terms(const DevScene& D, const int4 h1, int lit, V3f col, Dir wb_of, float pdf_b, float factor2, int li, V3f local, int& em1,
                                           int& em2, int& hot1, int& hot2, V3f& c1, V3f& c2)
 {
     float pdf_l = 0.0f;
@@ -438,7 +453,7 @@ __device__ __forceinline__ V3f area_terms(const DevScene& D, const int4 h1, int 
         if (mt.type == MCRT_LGHT)
         {
             const V3f ns1 = shading_normal(ts, float_of((uint32_t)h1.z), float_of((uint32_t)h1.w));
-            const V3f wb = ray_dir(rays, ib);
+            const V3f wb = wb_of();
             const float cosl = dot(ns1, -wb);
             if (!(cosl < 1e-6f))
             {
@@ -532,7 +547,8 @@ __global__ void k_resolve(PTArgs a, PTState S, int cur)
                 const int64_t hb = P + rf * P + bs;
                 V3f c1, c2;
                 local = area_terms(D, bs >= 0 ? S.hits[hb] : miss, li >= 0 ? reached(D, S.hits[h0], rays, h0, li) : -1,
-                                   col, rays, hb, r0.w, r1.w, li, local, em1, em2, hot1, hot2, c1, c2);
+                                   col, [&] { return ray_dir(rays, hb); }, r0.w, r1.w, li, local, em1, em2, hot1, hot2,
+                                   c1, c2);
                 if (ADJ)
                 {
                     const V3f dl = f3(S.delta[path]);
@@ -601,7 +617,7 @@ __device__ __forceinline__ void env_terms(const DevScene& D, uint64_t key, V3f n
     }
 }
 
-// Of a vertex at hit h of ray j: the ray's direction d, the hit point, the
+// Of a vertex at hit h of the ray (o, d): the hit point, the
 // shading normal and, where it has a next-event record and the scene area
 // lights, the BSDF-sampled next-event direction wb and whether that ray is
 // traced.  The BSDF-sampled ray adds a term only when its closest hit is an
@@ -612,14 +628,9 @@ __device__ __forceinline__ void env_terms(const DevScene& D, uint64_t key, V3f n
 // reaches none, and its terms are a miss's: it is not traced.  Rays with an
 // infinite inv_dir take the reference's NaN-prone sequential test and are
 // always traced.
-__device__ __forceinline__ void vertex_dirs(const DevScene& D, const RaySoA& rays, int64_t j, int4 h, const TriShade& ts,
-                                            bool want_rec, uint64_t key, V3f& d, V3f& phit, V3f& ns, V3f& wb,
-                                            bool& trace_wb)
+__device__ __forceinline__ void vertex_dirs(const DevScene& D, V3f o, V3f d, int4 h, const TriShade& ts, bool want_rec,
+                                            uint64_t key, V3f& phit, V3f& ns, V3f& wb, bool& trace_wb)
 {
-    const float4 ra = rays.od[j];
-    const float2 rb = rays.d[j];
-    const V3f o = f3(ra);
-    d = V3f{ra.w, rb.x, rb.y};
     const float t = float_of((uint32_t)h.y), u = float_of((uint32_t)h.z), v = float_of((uint32_t)h.w);
     phit = o + d * t;
     ns = shading_normal(ts, u, v);
@@ -737,7 +748,12 @@ __global__ __launch_bounds__(kShadeTPB) void k_shade(PTArgs a, PTState S, int cu
         // segment.
         V3f d = v3f(0.0f, 0.0f, 0.0f), phit = d, ns = d, wb = d;
         bool trace_wb = false;
-        if (act && h.x >= 0) vertex_dirs(D, rays, j, h, ts, want_rec, key, d, phit, ns, wb, trace_wb);
+        if (act && h.x >= 0)
+        {
+            V3f o;
+            load_ray(rays, j, o, d);
+            vertex_dirs(D, o, d, h, ts, want_rec, key, phit, ns, wb, trace_wb);
+        }
         // The path's throughput and whether its previous vertex was diffuse
         // are loaded before the slots too: their latency overlaps the slot
         // atomic.  The first vertex has unit throughput and no predecessor.
@@ -860,6 +876,83 @@ __global__ __launch_bounds__(kShadeTPB) void k_shade(PTArgs a, PTState S, int cu
     if (ADJ) hot_flush(a.one.D, acc, S.g_alb, S.g_em);
 }
 
+// The light sample of a vertex, as k_shade_direct emits it: whether its
+// shadow ray is traced, what it adds (x, c2: radiance, emission coefficient)
+// where it reaches triangle `tri`.
+struct Direct
+{
+    V3f wo = {0.0f, 0.0f, 0.0f}, x = {0.0f, 0.0f, 0.0f}, c2 = {0.0f, 0.0f, 0.0f};
+    float factor2 = 0.0f;
+    int li = -1, tri = -1, hot = -1;
+    bool want_sh = false;
+};
+// trace_wb: whether the BSDF-sampled ray is traced, so that the vertex's two
+// terms are summed in a record; set for a term that is not zero in the dark
+// (infinite or NaN colours or throughput), which is left to a record.
+template <bool ADJ>
+__device__ __forceinline__ Direct direct_light(const DevScene& D, uint64_t key, V3f phit, V3f ns, V3f col, V3f T,
+                                               bool& trace_wb)
+{
+    const V3f zero = v3f(0.0f, 0.0f, 0.0f);
+    Direct q;
+    V3f le = zero;
+    const LightSample ls = sample_area(D, key, phit, ns);
+    q.wo = ls.wo;
+    q.factor2 = ls.factor2;
+    q.li = ls.li;
+    bool reach = false;
+    if (q.li >= 0)
+    {
+        q.tri = D.lights[q.li].tri;
+        const float* tv = D.verts + 9 * (int64_t)q.tri;
+        const V3f v0 = ld3(tv), e1 = ld3(tv + 3) - v0, e2 = ld3(tv + 6) - v0;
+        RayPrep r;
+        r.ox = phit.x; r.oy = phit.y; r.oz = phit.z;
+        r.dx = q.wo.x; r.dy = q.wo.y; r.dz = q.wo.z;
+        float t, u, v;
+        if (mt(r, v0.x, v0.y, v0.z, e1.x, e1.y, e1.z, e2.x, e2.y, e2.z, D.det_eps, t, u, v) && t > kEpsRay &&
+            t < __builtin_inff())
+        {
+            const TriShade tl = D.shade[q.tri];
+            reach = !(dot(shading_normal(tl, u, v), -q.wo) < 0);
+            le = ld3(D.mats[tl.mat].rgb);
+            q.hot = tl.hot;
+        }
+    }
+    // area_terms with a missing BSDF-sampled ray, the light visible and not
+    const V3f none = zero + col * zero;
+    const float ip = 1.0f / kPi;
+    const V3f f = v3f(ip, ip, ip) * col;
+    const V3f lit = (f * le) * q.factor2, dark = (f * zero) * q.factor2;
+    q.want_sh = reach && !(lit.x == dark.x && lit.y == dark.y && lit.z == dark.z);
+    if (ADJ)  // the coefficient of the emission counts where the emission is zero, too
+    {
+        q.c2 = f * q.factor2;
+        q.want_sh = q.want_sh || (reach && !(q.c2.x == 0.0f && q.c2.y == 0.0f && q.c2.z == 0.0f));
+    }
+    q.x = T * (none + lit);
+    const V3f x0 = T * (q.li >= 0 ? none + dark : none);
+    if (!(x0.x == 0.0f && x0.y == 0.0f && x0.z == 0.0f)) trace_wb = true;
+    if (!ADJ && !trace_wb && q.x.x == 0.0f && q.x.y == 0.0f && q.x.z == 0.0f) q.want_sh = false;
+    return q;
+}
+
+// Continuation (Material::sample, demo_pt.cpp:645-650): the next direction;
+// T becomes the throughput behind the vertex, before the roulette's scale.
+__device__ __forceinline__ V3f continuation(const DevMaterial& m, uint64_t key, V3f d, V3f ns, V3f& T)
+{
+    const V3f col = ld3(m.rgb);
+    if (m.type == MCRT_GLSY)
+    {
+        float w;
+        const V3f nd = glossy_dir(-d, ns, m.gloss, rng_u01(key, 5), rng_u01(key, 6), w);
+        T = T * (col * w);
+        return nd;
+    }
+    T = T * col;
+    return lambert_dir(ns, rng_u01(key, 5), rng_u01(key, 6));
+}
+
 // One vertex of every live path in a render without an environment map.  The light sample comes before the workgroup takes its slots, with the
 // sampled triangle's own Moller-Trumbore test (the traversal's arithmetic on
 // the traversal's operands, so its t, u, v are those of a hit): a shadow ray
@@ -924,58 +1017,18 @@ __global__ __launch_bounds__(kShadeTPB) __attribute__((amdgpu_waves_per_eu(ADJ |
         const V3f zero = v3f(0.0f, 0.0f, 0.0f);
         V3f d = zero, phit = zero, ns = zero, wb = zero;
         bool trace_wb = false;
-        if (hit) vertex_dirs(D, rays, j, h, ts, want_rec, key, d, phit, ns, wb, trace_wb);
+        if (hit)
+        {
+            V3f o;
+            load_ray(rays, j, o, d);
+            vertex_dirs(D, o, d, h, ts, want_rec, key, phit, ns, wb, trace_wb);
+        }
         V3f T = f3(tq);
         const bool no_direct = k == 0 || !sp.nee || (bits_of(tq.w) & kDiffuseBit) == 0;
         const V3f col = ld3(mt.rgb);
-        V3f wo = zero, x = zero, c2 = zero;
-        float factor2 = 0.0f;
-        int li = -1, tri = -1, tri_hot = -1;
-        bool want_sh = false;
-        if (want_rec)
-        {
-            V3f le = zero;
-            LightSample ls = sample_area(D, key, phit, ns);
-            wo = ls.wo;
-            factor2 = ls.factor2;
-            li = ls.li;
-            bool reach = false;
-            if (li >= 0)
-            {
-                tri = D.lights[li].tri;
-                const float* tv = D.verts + 9 * (int64_t)tri;
-                const V3f v0 = ld3(tv), e1 = ld3(tv + 3) - v0, e2 = ld3(tv + 6) - v0;
-                RayPrep r;
-                r.ox = phit.x; r.oy = phit.y; r.oz = phit.z;
-                r.dx = wo.x; r.dy = wo.y; r.dz = wo.z;
-                float t, u, v;
-                if (mcrt::mt(r, v0.x, v0.y, v0.z, e1.x, e1.y, e1.z, e2.x, e2.y, e2.z, D.det_eps, t, u, v) &&
-                    t > kEpsRay && t < __builtin_inff())
-                {
-                    const TriShade tl = D.shade[tri];
-                    reach = !(dot(shading_normal(tl, u, v), -wo) < 0);
-                    le = ld3(D.mats[tl.mat].rgb);
-                    tri_hot = tl.hot;
-                }
-            }
-            // area_terms with a missing BSDF-sampled ray, the light visible and not
-            const V3f none = zero + col * zero;
-            const float ip = 1.0f / kPi;
-            const V3f f = v3f(ip, ip, ip) * col;
-            const V3f lit = (f * le) * factor2, dark = (f * zero) * factor2;
-            want_sh = reach && !(lit.x == dark.x && lit.y == dark.y && lit.z == dark.z);
-            if (ADJ)  // the coefficient of the emission counts where the emission is zero, too
-            {
-                c2 = f * factor2;
-                want_sh = want_sh || (reach && !(c2.x == 0.0f && c2.y == 0.0f && c2.z == 0.0f));
-            }
-            x = T * (none + lit);
-            const V3f x0 = T * (li >= 0 ? none + dark : none);
-            // a term that is not zero in the dark (infinite or NaN colours or
-            // throughput) is left to a record
-            if (!(x0.x == 0.0f && x0.y == 0.0f && x0.z == 0.0f)) trace_wb = true;
-            if (!ADJ && !trace_wb && x.x == 0.0f && x.y == 0.0f && x.z == 0.0f) want_sh = false;
-        }
+        Direct dl;
+        if (want_rec) dl = direct_light<ADJ>(D, key, phit, ns, col, T, trace_wb);
+        const bool want_sh = dl.want_sh;
         uint32_t cslot, sslot, bslot;
         block_slots(S.cnt[nxt], want_cont, want_sh, trace_wb, 1u, cslot, sslot, bslot);
         int alb_key = -1, em_key = -1, hot = -1;
@@ -998,23 +1051,23 @@ __global__ __launch_bounds__(kShadeTPB) __attribute__((amdgpu_waves_per_eu(ADJ |
         {
             // every later term carries this vertex's albedo once
             const V3f rest = f3(S.Ltot[p]) - f3(S.L[p]);
-            const V3f dl = f3(S.delta[p]);
+            const V3f de = f3(S.delta[p]);
             alb_key = h.x;
             hot = ts.hot;
-            g_alb = v3f(col.x > 0.0f ? dl.x * rest.x / col.x : 0.0f, col.y > 0.0f ? dl.y * rest.y / col.y : 0.0f,
-                        col.z > 0.0f ? dl.z * rest.z / col.z : 0.0f);
+            g_alb = v3f(col.x > 0.0f ? de.x * rest.x / col.x : 0.0f, col.y > 0.0f ? de.y * rest.y / col.y : 0.0f,
+                        col.z > 0.0f ? de.z * rest.z / col.z : 0.0f);
         }
         const RaySoA nr = S.rays[nxt];
         if (want_sh)
         {
             const int64_t r1 = a.P + (int64_t)sslot;
-            store_ray(nr, r1, phit, wo);
-            S.sh[nxt][sslot] = make_float4(x.x, x.y, x.z, float_of(trace_wb ? ~0u : p));
-            S.want[nxt][sslot] = (uint32_t)tri;
+            store_ray(nr, r1, phit, dl.wo);
+            S.sh[nxt][sslot] = make_float4(dl.x.x, dl.x.y, dl.x.z, float_of(trace_wb ? ~0u : p));
+            S.want[nxt][sslot] = (uint32_t)dl.tri;
             if (ADJ)
             {
-                const V3f g = (f3(S.delta[p]) * T) * c2;
-                S.shg[nxt][sslot] = make_float4(g.x, g.y, g.z, float_of((uint32_t)tri_hot));
+                const V3f g = (f3(S.delta[p]) * T) * dl.c2;
+                S.shg[nxt][sslot] = make_float4(g.x, g.y, g.z, float_of((uint32_t)dl.hot));
             }
             if (BATCH) S.rsid[nxt][r1] = sid;
         }
@@ -1023,28 +1076,14 @@ __global__ __launch_bounds__(kShadeTPB) __attribute__((amdgpu_waves_per_eu(ADJ |
             const int64_t r2 = 2 * a.P + (int64_t)bslot;
             float4* R = S.rec[nxt] + rec_words(2) * (int64_t)bslot;
             R[0] = make_float4(T.x, T.y, T.z, fmax_ref(dot(wb, ns), kEpsCos) / kPi);
-            R[1] = make_float4(col.x, col.y, col.z, factor2);
-            R[2] = make_float4(float_of(p), float_of((uint32_t)li), float_of(want_sh ? sslot : ~0u), 0.0f);
+            R[1] = make_float4(col.x, col.y, col.z, dl.factor2);
+            R[2] = make_float4(float_of(p), float_of((uint32_t)dl.li), float_of(want_sh ? sslot : ~0u), 0.0f);
             store_ray(nr, r2, phit, wb);
             if (BATCH) S.rsid[nxt][r2] = sid;
         }
         if (want_cont)
         {
-            // Continuation (Material::sample, demo_pt.cpp:645-650)
-            const V3f wi = -d;
-            V3f nd, weight;
-            if (mt.type == MCRT_GLSY)
-            {
-                float w;
-                nd = glossy_dir(wi, ns, mt.gloss, rng_u01(key, 5), rng_u01(key, 6), w);
-                weight = col * w;
-            }
-            else
-            {
-                nd = lambert_dir(ns, rng_u01(key, 5), rng_u01(key, 6));
-                weight = col;
-            }
-            T = T * weight;
+            const V3f nd = continuation(mt, key, d, ns, T);
             if (k >= sp.rr_start) T = T * (1.0f / sp.rr_prob);
             S.tq[nxt][cslot] = make_float4(T.x, T.y, T.z, float_of(p | (mt.type == MCRT_DIFF ? kDiffuseBit : 0u)));
             store_ray(nr, cslot, phit, nd);
@@ -1113,7 +1152,7 @@ __global__ void k_direct(PTArgs a, PTState S, int cur)
             const int64_t hb = 2 * a.P + m;
             const int lit = ss >= 0 && S.sprim[ss] == (int)S.want[cur][ss] ? S.sprim[ss] : -1;
             V3f c1, c2;
-            const V3f local = area_terms(D, S.hits[hb], lit, f3(r1), rays, hb, r0.w, r1.w, li,
+            const V3f local = area_terms(D, S.hits[hb], lit, f3(r1), [&] { return ray_dir(rays, hb); }, r0.w, r1.w, li,
                                          v3f(0.0f, 0.0f, 0.0f), em1, em2, hot1, hot2, c1, c2);
             const V3f T = f3(r0), x = T * local;
             if (!(x.x == 0.0f && x.y == 0.0f && x.z == 0.0f)) S.L[path] = f4(f3(S.L[path]) + x);
@@ -1131,6 +1170,132 @@ __global__ void k_direct(PTArgs a, PTState S, int cur)
         }
     }
     if (ADJ) hot_flush(a.one.D, acc, S.g_alb, S.g_em);
+}
+
+// Whole paths in one launch, for frames too small to fill the chip: there a
+// bounce's launches last as long as their longest ray, and the frame the sum
+// of these over the bounces, 30 launches; here it lasts as long as its longest
+// path.  A path has four lanes, which hold its state alike and shade alike;
+// lane 0 traces its continuation ray while lane 1 traces the previous vertex's
+// shadow ray and lane 2 its BSDF-sampled ray.  The arithmetic, and the order
+// in which a path's terms are added, are those of the wavefront kernels.
+// Wavefront -> this kernel, depth 8, one to four samples per pixel: 97x61 over
+// 5k triangles 524 -> 219 us; over 100k triangles 4k paths 807 -> 208, 16k 978
+// -> 288, 65k 1,155 -> 428, 131k 1,326 -> 668; over 1.25M triangles 131k paths
+// 2,138 -> 822; without light sampling (one lane in four at work) 131k paths
+// 574 -> 354 over 5k triangles, 1,287 -> 489 over 450k.  At 262k paths it still
+// gained 13% over 100k triangles, at 524k it lost 33%; 1M paths over 5k
+// triangles took 3.9 instead of 1.7 ms.  The limit is where every scene and
+// option measured still gains a third.
+constexpr int64_t kSmallPaths = int64_t(1) << 17;
+constexpr int kSmallLds = 16;  // the spill area suffices for scenes tuned to at most this depth
+__global__ __launch_bounds__(kWave) void k_small_paths(PTArgs a, float4* __restrict__ Lout, uint32_t per_wave)
+{
+    __shared__ uint32_t s_node[(kSmallLds + 1) * kWave];
+    __shared__ float s_lo[(kSmallLds + 1) * kWave];
+    const ScenePT& sp = a.one;
+    const DevScene& D = sp.D;
+    TraceStack st;
+    st.node = s_node;
+    st.lo = s_lo;
+    st.stride = kWave;
+    st.lane = threadIdx.x;
+    st.depth = kSmallLds;
+    st.spill = D.spill;
+    st.spill_lane = blockIdx.x * kWave + threadIdx.x;
+    st.spill_stride = (uint32_t)D.spill_lanes;
+    TraceCount cnt;
+    const int lane = threadIdx.x, role = lane & 3, lead = lane & ~3;
+    if ((uint32_t)(lane >> 2) >= per_wave) return;  // a path's lanes leave together
+    for (int64_t p = (int64_t)blockIdx.x * per_wave + (lane >> 2); p < a.P; p += (int64_t)gridDim.x * per_wave)
+    {
+        const int64_t pixel = a.pix0 + p / sp.spp;
+        const uint64_t sample = (uint64_t)(sp.sample_offset + p % sp.spp);
+        const V3f zero = v3f(0.0f, 0.0f, 0.0f);
+        V3f o, d, T = v3f(1.0f, 1.0f, 1.0f), L = zero;
+        camera_ray(sp, pixel, sample, o, d);
+        bool alive = true, no_direct = true, trace_wb = false;
+        // of the previous vertex: its point, light sample and, for a record,
+        // throughput, colour and the BSDF-sampled direction with its pdf
+        Direct dl;
+        V3f pt = o, Tr = T, cr = zero, wb = zero;
+        float pdf_b = 0.0f;
+        for (int k = 0;; k++)
+        {
+            int4 h = make_int4(-1, 0, 0, 0);
+            if (role == 0 ? alive : role == 1 ? dl.want_sh : role == 2 && trace_wb)
+            {
+                const V3f ro = role == 0 ? o : pt, rd = role == 0 ? d : role == 1 ? dl.wo : wb;
+                RayPrep rp = prep_ray(ro.x, ro.y, ro.z, rd.x, rd.y, rd.z, kSegTmin);
+                node_margin(rp, D.node_span);
+                Tracer<false, false, false> tr;
+                tr.start(rp, __builtin_inff());
+                while (!tr.step(D, st, cnt)) {}
+                float t, u, v;
+                h.x = tr.result(t, u, v);
+                h.y = (int)bits_of(t);
+                h.z = (int)bits_of(u);
+                h.w = (int)bits_of(v);
+            }
+            const int sprim = __shfl(h.x, lead + 1);
+            const int4 hb = make_int4(__shfl(h.x, lead + 2), __shfl(h.y, lead + 2), __shfl(h.z, lead + 2),
+                                      __shfl(h.w, lead + 2));
+            h = make_int4(__shfl(h.x, lead), __shfl(h.y, lead), __shfl(h.z, lead), __shfl(h.w, lead));
+            // next-event terms of the previous vertex (k_direct)
+            const bool reached_light = dl.want_sh && sprim == dl.tri;
+            if (trace_wb)
+            {
+                int em1, em2, hot1, hot2;
+                V3f c1, c2;
+                const V3f x = Tr * area_terms(D, hb, reached_light ? dl.tri : -1, cr, [&] { return wb; }, pdf_b,
+                                              dl.factor2, dl.li, zero, em1, em2, hot1, hot2, c1, c2);
+                if (!(x.x == 0.0f && x.y == 0.0f && x.z == 0.0f)) L = L + x;
+            }
+            else if (reached_light)
+                L = L + dl.x;
+            dl = Direct();
+            trace_wb = false;
+            // the vertex (k_shade_direct)
+            if (k > sp.max_depth || !alive || h.x < 0) break;
+            alive = false;
+            const TriShade ts = D.shade[h.x];
+            const DevMaterial m = D.mats[ts.mat];
+            const V3f col = ld3(m.rgb);
+            uint64_t key = 0;
+            bool want_rec = false;
+            if (m.type != MCRT_LGHT)
+            {
+                key = rng_key(sp.seed, (uint64_t)pixel, sample, (uint32_t)k);
+                want_rec = sp.nee && m.type == MCRT_DIFF && D.nlights > 0;
+                alive = !(k >= sp.max_depth) && !(k >= sp.rr_start && rng_u01(key, 7) >= sp.rr_prob);
+            }
+            V3f ns;
+            vertex_dirs(D, o, d, h, ts, want_rec, key, pt, ns, wb, trace_wb);
+            if (m.type == MCRT_LGHT)
+            {
+                if (no_direct && dot(d, ns) < 0) L = L + T * col;
+                break;
+            }
+            if (want_rec)
+            {
+                dl = direct_light<false>(D, key, pt, ns, col, T, trace_wb);
+                Tr = T;
+                cr = col;
+                pdf_b = fmax_ref(dot(wb, ns), kEpsCos) / kPi;
+            }
+            if (alive)
+            {
+                const V3f nd = continuation(m, key, d, ns, T);
+                if (k >= sp.rr_start) T = T * (1.0f / sp.rr_prob);
+                no_direct = !sp.nee || m.type != MCRT_DIFF;
+                o = pt;
+                d = nd;
+            }
+            else if (!dl.want_sh && !trace_wb)
+                break;
+        }
+        if (role == 0) Lout[p] = make_float4(L.x, L.y, L.z, 0.0f);
+    }
 }
 
 // Adjoint seed: keep pass 1's radiance and form dLoss/dL of each path
@@ -1408,7 +1573,15 @@ int render_scene(mcrt_scene* s, StreamRes* r, const mcrt_render_params* prm, flo
         PTState S = state_of(r, a.P, adj != nullptr, rs);
         S.g_alb = adj ? adj->d_albedo : nullptr;
         S.g_em = adj ? adj->d_emission : nullptr;
-        bounce_loop<false, false>(D, S, a, prm->max_depth, cus, st);
+        if (rs == 2 && a.P <= kSmallPaths && D.lds_depth <= kSmallLds && !D.big)
+        {
+            // spread over the waves a small traversal launch uses, at most 16 paths to a wave
+            const int64_t per = std::min<int64_t>(kWave / 4, (a.P + kSpreadWaves - 1) / kSpreadWaves);
+            const int64_t blocks = std::min<int64_t>((a.P + per - 1) / per, D.spill_lanes / kWave);
+            hipLaunchKernelGGL(k_small_paths, dim3((unsigned)blocks), dim3(kWave), 0, st, a, S.L, (uint32_t)per);
+        }
+        else
+            bounce_loop<false, false>(D, S, a, prm->max_depth, cus, st);
         if (adj)
         {
             hipLaunchKernelGGL(k_delta, (grid_of<k_delta>(a.P, cus)), dim3(kTPB), 0, st, S, a, adj->dfilm,

@@ -249,4 +249,28 @@ def test_render_bit_exact_extreme_terms(ctx, what):
     d = scenes.SceneData(d.tris, normals, d.tri_mat, d.mat_type, rgb, d.mat_gloss)
     kw = dict(spp=4, max_depth=4, rr_start=2, rr_prob=0.8, seed=3, nee=True)
     print(f"[extreme terms: {what}]", flush=True)
-    _compare(what, gpu_render(ctx, d, 40, 33, **kw), oracle_render(d, 40, 33, **kw))
+    want = oracle_render(d, 40, 33, **kw)
+    _compare(what, gpu_render(ctx, d, 40, 33, **kw), want)
+    # a stack depth that the one-launch kernel of small frames does not take
+    s = d.to_scene(ctx, width=40, height=33)
+    s.set_tuning(pt_trace_lds_depth=24)
+    _compare(what + ", wavefront", s.render(**kw), want)
+
+
+@pytest.mark.parametrize("w,h,spp", [(1, 1, 1), (3, 1, 1), (31, 33, 2), (64, 32, 1), (683, 3, 1), (128, 128, 8),
+                                     (129, 128, 8)])
+def test_small_frames_equal_wavefront(ctx, w, h, spp):
+    """The one-launch kernel of small frames against the wavefront kernels
+    (taken with a 24-entry stack, and above 2^17 paths), bit for bit, at one
+    path, partial waves, the spread's edges and its largest size, glossy and
+    two lights' worth of terms, next-event estimation on and off."""
+    from mcrt_amd import scenes
+    d = scenes.cornell_displaced(sub=3, phong_frac=0.4)
+    s = d.to_scene(ctx, width=w, height=h)
+    for nee in (True, False):
+        kw = dict(spp=spp, max_depth=7, rr_start=2, rr_prob=0.8, seed=5, nee=nee)
+        print(f"[small frame {w}x{h}x{spp} nee={nee}]", flush=True)
+        s.set_tuning(pt_trace_lds_depth=8)
+        a = s.render(**kw)
+        s.set_tuning(pt_trace_lds_depth=24)
+        _compare(f"{w}x{h}x{spp} nee={nee}", a, s.render(**kw))
