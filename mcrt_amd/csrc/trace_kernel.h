@@ -30,12 +30,17 @@
 // makes them.  On the 100k-triangle sphere (claims of 128 before -> now):
 // 1,000 rays over 5k triangles 70 -> 38 us, 131k rays 165 -> 137, 400k
 // 262 -> 171, 1M 341 -> 237, 2M 400 -> 321; 500k any-hit rays 299 -> 200;
-// the 97x61 one-sample frame 1,087 -> 634 us.  At 4M rays (more than
-// kSpreadRays per wave) the two measured alike, and at 16M fixed windows
-// lose: waves that draw long rays end late.  kSpreadWaves 256 / 1,024 /
+// the 97x61 one-sample frame 1,087 -> 634 us.  kSpreadWaves 256 / 1,024 /
 // 4,096 / 8,192 instead of 2,048: 109 / 106 / 102 / 105 against 101 us at
 // 20k rays, the frame 720 / 659 / 615 / 610 against 635; windows of 64 or
 // 256 were 2-5% slower at 700k to 1M rays.
+// kSpreadRays 512 instead of 256, with steps that take less time against the
+// same counters: 2.4M rays over 100k triangles 361 -> 282 us, 4.1M over the
+// 1.3M-triangle mesh 606 -> 492, a 600x600x9 frame 4.70 -> 4.44 ms; with
+// 1,024 the sky frame lost 5% and an adjoint step 2%, as waves that draw long
+// rays end late.  A query in origin-cell order takes claims at any size: its
+// slices keep an XCD in one part of the tree (1.1M to 1.7M rays of the
+// 2M-triangle soup 5-9% faster, 3.6M rays a fifth).
 //
 // Two ray sources:
 //   * SEG = kQuery: rays[0, n) with n known to the host;
@@ -58,7 +63,7 @@ constexpr uint32_t kClaim = 128;
 // of the 2M-triangle soup 1,475 -> 1,409, its 8M incoherent rays 3,728 ->
 // 3,673 (3 instead of 4: 1,476 / 1,417 / 3,669).
 constexpr int kLeafShare = 4;
-constexpr uint32_t kSpreadRays = 256;    // most rays per wave of a launch with fixed windows
+constexpr uint32_t kSpreadRays = 512;    // most rays per wave of a launch with fixed windows
 constexpr uint32_t kSpreadWaves = 2048;  // waves a small launch is spread over
 constexpr uint32_t kSpreadWindow = 128;  // widest window while fewer waves than the grid's suffice
 // Word of a segment-mode count array holding the third segment's size (on
@@ -149,7 +154,7 @@ __global__ __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(
     // claim bookkeeping stays in scalar registers instead of being shuffled
     // through the LDS crossbar into vector registers.
     uint32_t ahead = 0;  // lane 0: offset of the requested next window in slice sl
-    if (total <= gridDim.x * kSpreadRays)
+    if (total <= gridDim.x * kSpreadRays && order == nullptr)
     {
         // a fixed window; past its end the wave finds its slice, the last
         // one left to try, used up

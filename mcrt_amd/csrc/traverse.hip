@@ -165,14 +165,15 @@ template <bool ANY, bool COUNT>
 hipError_t launch(const DevScene& s, const float* rays, int64_t n, void* hits, uint8_t* occ, uint64_t* counters,
                   hipStream_t stream)
 {
+    const bool order = s.order != nullptr && s.reorder_rays > 0 && n >= s.reorder_rays;
     // kernels, not hipMemsetAsync, so a caller may capture the query in a
     // graph; a launch with fixed windows reads no counters
-    if (n > trace_blocks(s, n) * (int64_t)kSpreadRays)
+    if (order || n > trace_blocks(s, n) * (int64_t)kSpreadRays)
         hipLaunchKernelGGL(k_wq_reset, dim3(1), dim3(64), 0, stream, s.wq);
     const float4* r4 = reinterpret_cast<const float4*>(rays);
     int4* h4 = reinterpret_cast<int4*>(hits);
     unsigned long long* c = reinterpret_cast<unsigned long long*>(counters);
-    if (s.order != nullptr && s.reorder_rays > 0 && n >= s.reorder_rays)
+    if (order)
     {
         hipLaunchKernelGGL(k_cell_reset, dim3(1), dim3(1024), 0, stream, s.cell_work);
         hipLaunchKernelGGL(k_cell_sample, dim3(1), dim3(1024), 0, stream, s, r4, (uint32_t)n);

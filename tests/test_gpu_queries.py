@@ -260,9 +260,10 @@ def test_ties_and_degenerate_triangles(ctx):
     s.close()
 
 
-@pytest.mark.parametrize("n", [2, 63, 2047, 2049, 3000, 256 * 128 + 1, 256 * 256 - 1, 256 * 256, 256 * 256 + 1])
+@pytest.mark.parametrize("n", [2, 63, 2047, 2049, 3000, 256 * 128 + 1, 256 * 256 - 1, 256 * 256, 256 * 256 + 1,
+                               256 * 512 - 1, 256 * 512, 256 * 512 + 1])
 def test_fixed_windows_and_claims_bit_exact(ctx, n):
-    """Launches with one fixed window per wave (at most 256 rays per wave of
+    """Launches with one fixed window per wave (at most 512 rays per wave of
     the grid, here 256 waves) and with claimed windows, at the edges of the
     window rule: every ray is traced once, closest and any hit."""
     import mcrt_amd
