@@ -44,7 +44,7 @@ static_assert(sizeof(WNode) == 128, "WNode must be 128 bytes");
 // The node the kernels read: a WNode with its child boxes quantised to 8
 // bits per plane, rounded outwards, in 64 B (four 16 B rows):
 //   row 0: origin x, y, z (float) | scale exponents ex | ey << 8 | ez << 16
-//          | child count << 24
+//          | child count << 24 (on the device a mask of as many low bits)
 //   row 1: child[4] (links as in WNode)
 //   row 2: lo_x, hi_x, lo_y, hi_y   (byte c of each word = child c)
 //   row 3: lo_z, hi_z, rank_lo, rank_hi

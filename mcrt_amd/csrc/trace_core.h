@@ -181,9 +181,9 @@ MCRT_HD bool qslab_c(const RayPrep& r, uint32_t nx, uint32_t fx, uint32_t ny, ui
                      uint32_t nz, uint32_t fz, float ax, float ay, float az, float nbx, float fbx, float nby,
                      float fby, float nbz, float fbz, int shift, float R1, float& lo)
 {
-    // computed for every slot: an empty slot's planes are inverted, and its
-    // link leads to a reference that nothing hits, should a node be so small
-    // against the margin that they pass (device_records, wide.cpp)
+    // computed for every slot: an empty slot's planes are inverted, and where
+    // they pass all the same the node's mask of children drops the slot
+    // (device_records, wide.cpp)
     const float t0x = __builtin_fmaf((float)((nx >> shift) & 0xffu), ax, nbx);
     const float t1x = __builtin_fmaf((float)((fx >> shift) & 0xffu), ax, fbx);
     const float t0y = __builtin_fmaf((float)((ny >> shift) & 0xffu), ay, nby);
@@ -373,7 +373,12 @@ struct Tracer
             // near-first order finds occluders sooner than slot order.)
             const uint32_t rk = (r.oct_hi ? qb.w : qb.z) >> r.oct_shift;
             const uint32_t r0 = rk & 3u, r1 = (rk >> 2) & 3u, r2 = (rk >> 4) & 3u, r3 = (rk >> 6) & 3u;
-            const uint32_t m = ((uint32_t)p0 << r0) | ((uint32_t)p1 << r1) | ((uint32_t)p2 << r2) | ((uint32_t)p3 << r3);
+            // An exact ray's tests pass for empty slots, too, and those of a
+            // node that is small against the margin may; the node's mask of
+            // children takes them out, since the stack's bound counts children
+            // only.  (Empty slots are last in every order: device_records.)
+            const uint32_t m =
+                (((uint32_t)p0 << r0) | ((uint32_t)p1 << r1) | ((uint32_t)p2 << r2) | ((uint32_t)p3 << r3)) & (hd.w >> 24);
             if (m != 0)
             {
                 const uint32_t first = (uint32_t)__builtin_ctz(m);
@@ -387,29 +392,32 @@ struct Tracer
                     // every row up to the nearest child's, one above the
                     // entries kept, is in LDS: four unconditional writes,
                     // the nearest child's a dead entry, those of failing
-                    // slots into the discard row
+                    // slots into the discard row.  An empty slot that passed
+                    // is written at row sp, so before the children, the
+                    // farthest of which belongs there.
                     const uint32_t dis = st.off(st.depth);
                     if (ANY)
                     {
-                        st.put_node(p0 ? st.off(i0) : dis, ch.x);
-                        st.put_node(p1 ? st.off(i1) : dis, ch.y);
-                        st.put_node(p2 ? st.off(i2) : dis, ch.z);
                         st.put_node(p3 ? st.off(i3) : dis, ch.w);
+                        st.put_node(p2 ? st.off(i2) : dis, ch.z);
+                        st.put_node(p1 ? st.off(i1) : dis, ch.y);
+                        st.put_node(p0 ? st.off(i0) : dis, ch.x);
                     }
                     else
                     {
-                        st.put(p0 ? st.off(i0) : dis, ch.x, l0);
-                        st.put(p1 ? st.off(i1) : dis, ch.y, l1);
-                        st.put(p2 ? st.off(i2) : dis, ch.z, l2);
                         st.put(p3 ? st.off(i3) : dis, ch.w, l3);
+                        st.put(p2 ? st.off(i2) : dis, ch.z, l2);
+                        st.put(p1 ? st.off(i1) : dis, ch.y, l1);
+                        st.put(p0 ? st.off(i0) : dis, ch.x, l0);
                     }
                 }
                 else
                 {
-                    if (p0 && r0 != first) st.push(i0, ch.x, l0);
-                    if (p1 && r1 != first) st.push(i1, ch.y, l1);
-                    if (p2 && r2 != first) st.push(i2, ch.z, l2);
-                    if (p3 && r3 != first) st.push(i3, ch.w, l3);
+                    const uint32_t rest = m & (m - 1u);  // without the nearest
+                    if ((rest >> r0) & 1u) st.push(i0, ch.x, l0);
+                    if ((rest >> r1) & 1u) st.push(i1, ch.y, l1);
+                    if ((rest >> r2) & 1u) st.push(i2, ch.z, l2);
+                    if ((rest >> r3) & 1u) st.push(i3, ch.w, l3);
                 }
                 sp += c - 1;
                 return false;

@@ -348,12 +348,60 @@ float qnode_span(const std::vector<QNode>& q)
     return f;
 }
 
+namespace
+{
+// Moves a node's n children to slots 0..n-1 and to the first n positions of
+// every octant's order, keeping their order in both.  (Builders leave nodes
+// like this but for leaves without references.)
+void pack_children(QNode& q, int n)
+{
+    const uint32_t rest = n < 4 ? 0x01010101u * (0xffu & (0xffu << (2 * n))) : 0u;  // rank fields of slots n..3
+    bool packed = ((q.rank_lo ^ 0xe4e4e4e4u) & rest) == 0 && ((q.rank_hi ^ 0xe4e4e4e4u) & rest) == 0;
+    for (int c = 0; c < n; c++) packed = packed && q.child[c] != MCRT_CHILD_EMPTY;
+    if (packed) return;
+    int from[4], k = 0, e = n;
+    for (int c = 0; c < 4; c++) from[q.child[c] != MCRT_CHILD_EMPTY ? k++ : e++] = c;
+    QNode r = q;
+    r.rank_lo = r.rank_hi = 0;
+    for (uint32_t QNode::*w : {&QNode::q_lo_x, &QNode::q_hi_x, &QNode::q_lo_y, &QNode::q_hi_y, &QNode::q_lo_z,
+                               &QNode::q_hi_z})
+    {
+        r.*w = 0;
+        for (int c = 0; c < 4; c++) r.*w |= ((q.*w >> (8 * from[c])) & 0xffu) << (8 * c);
+    }
+    for (int c = 0; c < 4; c++) r.child[c] = q.child[from[c]];
+    for (int o = 0; o < 8; o++)
+    {
+        const uint32_t b = (o < 4 ? q.rank_lo : q.rank_hi) >> (8 * (o & 3));
+        uint32_t byte = 0;
+        for (int c = 0; c < 4; c++)
+        {
+            uint32_t pos = (uint32_t)c;  // of a child: the children before it
+            if (c < n)
+            {
+                pos = 0;
+                for (int d = 0; d < n; d++)
+                    pos += ((b >> (2 * from[d])) & 3u) < ((b >> (2 * from[c])) & 3u) ? 1u : 0u;
+            }
+            byte |= pos << (2 * c);
+        }
+        (o < 4 ? r.rank_lo : r.rank_hi) |= byte << (8 * (o & 3));
+    }
+    q = r;
+}
+}  // namespace
+
 bool device_records(const WideBVH& wb, std::vector<QNode>& nodes_out)
 {
     const uint64_t nq = wb.qnodes.size() + 1;  // and the reference of empty slots
     if (nq + wb.refs.size() > (uint64_t)MCRT_LEAF_REF_MASK + 1u) return false;
     nodes_out = wb.qnodes;
     for (QNode& q : nodes_out)
+    {
+        int n = 0;
+        for (int c = 0; c < 4; c++) n += q.child[c] != MCRT_CHILD_EMPTY ? 1 : 0;
+        pack_children(q, n);
+        q.exps = (q.exps & 0xffffffu) | (((1u << n) - 1u) << 24);
         for (int c = 0; c < 4; c++)
         {
             const uint32_t byte = 0xffu << (8 * c);
@@ -366,6 +414,7 @@ bool device_records(const WideBVH& wb, std::vector<QNode>& nodes_out)
             else if (q.child[c] & MCRT_CHILD_LEAF)
                 q.child[c] += (uint32_t)nq;  // stays below bit 29: every reference index + nq fits
         }
+    }
     // an inverted infinite box around a triangle without area
     WRef none;
     std::memset(&none, 0, sizeof(none));

@@ -39,11 +39,14 @@ void optimize_wide(WideBVH& wb);
 float qnode_span(const std::vector<QNode>& q);
 
 // The device's record array, nodes then references (layout.h): the QNodes
-// with every leaf link rebased, then one record for empty slots.  There an
-// empty slot has inverted planes (no test for it in the kernels' node step;
+// with every leaf link rebased and, in place of the child count, a mask of the
+// positions in an octant's order that children take (the first ones: empty
+// slots go last), then one record for empty slots.  There an empty slot has inverted planes (no test for it in the kernels' node step;
 // 16M rays of the 1.3M-triangle mesh 1,409 -> 1,389 us, 1,000 rays over 5k
 // triangles 32.4 -> 30.1) and links to a reference with an inverted infinite
-// box and a triangle without area, which no ray hits.  Writes these records
+// box and a triangle without area, which no ray hits.  The mask keeps a slot
+// whose inverted planes pass (an exact ray's do) from being visited at all.
+// It costs the closest-hit launch above 0.6%, the 1,000 rays 1 us.  Writes these records
 // into `nodes_out` (the references follow them unchanged).  Returns false
 // when the records do not fit the 29-bit link index.
 bool device_records(const WideBVH& wb, std::vector<QNode>& nodes_out);

@@ -98,6 +98,7 @@ def hostemu():
         "emu_build": (P, [P, LL, I]),
         "emu_digest": (U64, [P, P]),
         "emu_optimize": (None, [P, P]),
+        "emu_stack_use": (I, [P, P, LL, I]),
         "emu_free": (None, [P]),
         "emu_set_eps": (None, [P, F]),
         "emu_margin_check": (None, [LL, U64, F, P, P]),

@@ -207,6 +207,46 @@ extern "C" void emu_trace(void* h, const float* rays, long long n, int* hits, un
     if (counters) { counters[0] = cn; counters[1] = cr; counters[2] = ct; }
 }
 
+// The most stack entries a traversal of any of the rays ever holds, every
+// entry in a spill area larger than the bound.
+extern "C" int emu_stack_use(void* h, const float* rays, long long n, int any)
+{
+    Emu* e = (Emu*)h;
+    DevScene S;
+    S.nodes = e->recs.data();
+    S.stack_bound = e->wb.stack_bound;
+    S.node_span = qnode_span(e->wb.qnodes);
+    S.det_eps = e->det_eps;
+    uint32_t sn = 0;
+    float sl = 0.0f;
+    const uint64_t unused = ~0ull;
+    std::vector<uint64_t> spill(4 * (size_t)e->wb.depth + 8, unused);
+    TraceStack st;
+    st.node = &sn;
+    st.lo = &sl;
+    st.stride = 1;
+    st.lane = 0;
+    st.depth = 0;
+    st.spill = spill.data();
+    st.spill_lane = 0;
+    st.spill_stride = 1;
+    for (long long i = 0; i < n; i++)
+    {
+        const float* r = rays + 8 * i;
+        RayPrep rp = prep_ray(r[0], r[1], r[2], r[4], r[5], r[6], r[3]);
+        TraceCount c;
+        float t, u, v;
+        if (any)
+            trace<true, true>(S, st, rp, r[7], t, u, v, c);
+        else
+            trace<false, true>(S, st, rp, r[7], t, u, v, c);
+    }
+    int used = 0;
+    for (size_t k = 0; k < spill.size(); k++)
+        if (spill[k] != unused) used = (int)k + 1;
+    return used;
+}
+
 // The node-test margin (trace_core.h: node_margin) against the reference's
 // slab arithmetic on single planes: n random cases of node origin, scale
 // 2^k, plane code, ray origin and direction (magnitudes from tiny to huge,

@@ -311,3 +311,23 @@ def test_special_rays_equal_oracle(emu, which):
     assert np.array_equal(hits[:, 1:].view(np.uint32), tuv.view(np.uint32))
     occ, _ = e.trace(rays, any_hit=True)
     assert np.array_equal(occ, (prim >= 0).astype(np.uint8))
+
+
+@pytest.mark.parametrize("n", [1, 2, 4, 60, 968])
+@pytest.mark.parametrize("any_hit", [False, True])
+@pytest.mark.parametrize("optimised", [False, True])
+def test_exact_rays_keep_the_stack_bound(emu, n, any_hit, optimised):
+    """A ray with an infinite 1 / d passes every node test, so it holds the
+    most entries: no more than the bound the spill area is sized with, which
+    counts a node's children and not its empty slots."""
+    tris = _libs.debug_mesh() if n == 968 else np.random.default_rng(n).random((n, 9), dtype=np.float32)
+    rays = _libs.random_rays(tris, 512, seed=4)
+    rays[np.arange(512), 4 + np.arange(512) % 3] = 1e-42
+    rays[:, 7] = 3e38
+    e = Emu(tris)
+    st = np.zeros(8, np.int64)
+    if optimised:
+        e.L.emu_optimize(e.h, ptr(st))
+    else:
+        st = e.digest()[1]
+    assert e.L.emu_stack_use(e.h, ptr(rays), rays.shape[0], 1 if any_hit else 0) <= st[6]
