@@ -9,22 +9,27 @@
 //     extend             one traversal launch over the compacted
 //                        continuation rays AND the next-event rays of
 //                        vertex k-1 (segment counts read on the device)
-//     resolve            next-event contributions of vertex k-1 (MIS),
+//     direct             next-event contributions of vertex k-1 (MIS),
 //                        added before anything of vertex k, as in the
 //                        reference's accumulation order
-//     shade (k <= max)   emitter hit or escape to the environment,
-//                        next-event rays at diffuse vertices, BSDF
-//                        continuation, Russian roulette
+//     shade (k <= max)   emitter hit, next-event rays at diffuse vertices
+//                        that can add light, BSDF continuation, Russian
+//                        roulette
 //   accumulate           per-pixel sum in sample order of each path's
 //                        radiance (NaN -> 0, clamp >= 0) x (1/spp)
 // Every kernel is grid-strided over a fixed grid and reads its work count
 // from device memory, so the whole chunk is launch-only (graph-capturable).
+// With an environment map resolve takes direct's place and shade also adds
+// what escapes to the map (k_resolve, k_shade; without one k_direct and
+// k_shade_direct, whose records hold the finished next-event terms).  A frame
+// of few paths is one launch instead (k_small_paths).
 //
-// A diffuse vertex's next-event record has rs rays: the BSDF-sampled ray
-// and the light-sampled shadow ray of the area lights, and, with an
-// environment map (rs = 4), the shadow rays of its two environment samples
-// (one drawn from the map's pdf, one from the cosine lobe; demo_pt.cpp:
-// 421-499, 564-589).  The record's other rays sit at its slots; the
+// Without an environment map a next-event record is written only for a
+// vertex whose light-sampled term is not zero, and its shadow ray with it.
+// With one, every diffuse vertex's record has rs = 4 rays: the BSDF-sampled
+// ray and the light-sampled shadow ray of the area lights, and the shadow
+// rays of its two environment samples (one drawn from the map's pdf, one from
+// the cosine lobe; demo_pt.cpp:421-499, 564-589).  The record's other rays sit at its slots; the
 // BSDF-sampled ray is traced only where it can reach an emitter and then
 // goes to a compacted segment of its own, its slot kept with the record.  A
 // ray a scene does not need has a zero direction, which every box rejects.
@@ -953,8 +958,9 @@ __device__ __forceinline__ V3f continuation(const DevMaterial& m, uint64_t key, 
     return lambert_dir(ns, rng_u01(key, 5), rng_u01(key, 6));
 }
 
-// One vertex of every live path in a render without an environment map.  The light sample comes before the workgroup takes its slots, with the
-// sampled triangle's own Moller-Trumbore test (the traversal's arithmetic on
+// One vertex of every live path in a render without an environment map.  The
+// light sample comes before the workgroup takes its slots, with the sampled
+// triangle's own Moller-Trumbore test (the traversal's arithmetic on
 // the traversal's operands, so its t, u, v are those of a hit): a shadow ray
 // exists only where its triangle can be hit, faces the vertex and adds
 // something, and what it adds is known up to visibility.  So most vertices
@@ -967,8 +973,9 @@ __device__ __forceinline__ V3f continuation(const DevMaterial& m, uint64_t key, 
 // before): 76.3 -> 64.3 ms, the extend launches 52 -> 44.2 ms (a quarter of
 // the shadow rays gone: lights behind the surface were traced for a zero
 // term), next-event sums 8.3 -> 4.2 ms, this kernel 15.2 -> 14.8 ms at 76
-// instead of 86 registers (6 waves per SIMD).  Bound by the latency of its
-// dependent loads (path, hit, triangle, material) and by its stores.
+// instead of 86 registers (6 waves per SIMD).  Bound by the workgroups' slot
+// atomics (kShadeTPB: 14.8 -> 10.6 ms), then by the latency of its dependent
+// loads (path, hit, triangle, material) and by its stores: 3.0 TB/s.
 template <bool ADJ, bool BATCH>
 __global__ __launch_bounds__(kShadeTPB) __attribute__((amdgpu_waves_per_eu(ADJ || BATCH ? 5 : 6, 8))) void k_shade_direct(
     PTArgs a, PTState S, int cur, int k)

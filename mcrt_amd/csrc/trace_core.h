@@ -275,8 +275,8 @@ struct TraceCount
     uint32_t nodes = 0, refs = 0, tris = 0;
 };
 
-// What bounds it: vector instructions (88% of the issue slots on 16M rays of
-// the 1.3M-triangle mesh, 45 wave instructions a ray) and, behind them, the
+// What bounds it: vector instructions (93% of the issue slots on 16M rays of
+// the 1.3M-triangle mesh, 43 wave instructions a ray) and, behind them, the
 // scalar mask instructions of the branches.  The node step therefore has no
 // branch but the stack's: the three range comparisons of a child are one (max
 // and min with the ray's limits), rays that need the exact tests pass every
